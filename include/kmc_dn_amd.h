@@ -93,7 +93,7 @@ int kmc_simulate_discrete(int64_t N, int64_t P, double nu, double kT, double I_0
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  Same arguments, kernel and results;
  * it calls no hipMalloc/hipFree and no allocating routine: every device buffer
- * is carved from one static scratch array per device (about 2.1 MiB, held
+ * is carved from one static scratch array per device (about 4.1 MiB, held
  * until the process ends).  Limits: S = N + P <= KMC_NOALLOC_MAX_SITES, and
  * with replayed uniforms or event/total logs at most KMC_NOALLOC_MAX_LOGGED_HOPS
  * hops (KMC_ERR_LIMIT beyond).  Calls on one device share its scratch and keep

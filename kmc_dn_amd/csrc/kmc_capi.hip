@@ -32,7 +32,9 @@ __global__ void kmc_queue_reset_kernel(int32_t*);
 __global__ void kmc_fill_zero_kernel(double*, int64_t);
 __global__ void kmc_eset_scatter_kernel(const EsetDev*, const int32_t*, const int32_t*, const double*,
                                         const double*, int64_t);
-size_t plain_lds_bytes(int S, int N, bool stage);
+size_t plain_lds_bytes(int S, int N, int slots, bool stage);
+size_t plain_state_bytes(int S, int N);
+int plain_pairs(int S, int N);
 size_t batch_lds_bytes(bool bt, int C, int W, int S, int N, int P);
 size_t pos_lds_bytes(int C, int W);
 size_t store_lds_bytes(int W, int slots);
@@ -58,7 +60,7 @@ constexpr size_t NOALLOC_TABLE = (size_t)KMC_NOALLOC_MAX_SITES * KMC_NOALLOC_MAX
 constexpr size_t NOALLOC_ALIGN = 256;
 constexpr size_t noalloc_up(size_t x) { return (x + NOALLOC_ALIGN - 1) & ~(NOALLOC_ALIGN - 1); }
 // carve-up (byte offsets): descriptors, E, V, d, tc, ird, invd, traffic,
-// se_out, occ_time, uniforms, events, totals
+// se_out, occ_time, uniforms, events, totals, state records
 constexpr size_t NA_DESC = 0;
 constexpr size_t NA_E = noalloc_up(NA_DESC + 1024);
 constexpr size_t NA_V = noalloc_up(NA_E + sizeof(double) * KMC_NOALLOC_MAX_SITES);
@@ -72,7 +74,9 @@ constexpr size_t NA_OT = noalloc_up(NA_SE + sizeof(double) * KMC_NMAX);
 constexpr size_t NA_U = noalloc_up(NA_OT + sizeof(double) * KMC_NMAX);
 constexpr size_t NA_EV = NA_U + sizeof(double) * 2 * KMC_NOALLOC_MAX_LOGGED_HOPS;
 constexpr size_t NA_TOT = noalloc_up(NA_EV + sizeof(int32_t) * KMC_NOALLOC_MAX_LOGGED_HOPS);
-constexpr size_t NOALLOC_BYTES = noalloc_up(NA_TOT + sizeof(double) * KMC_NOALLOC_MAX_LOGGED_HOPS);
+constexpr size_t NA_STATES = noalloc_up(NA_TOT + sizeof(double) * KMC_NOALLOC_MAX_LOGGED_HOPS);
+constexpr size_t NOALLOC_STATES = (size_t)2 << 20;   // state records: 64 of the largest network's
+constexpr size_t NOALLOC_BYTES = NA_STATES + NOALLOC_STATES;
 static_assert(sizeof(LayoutDev) + sizeof(EsetDev) + sizeof(TrajDev) + sizeof(TrajOut) + 64 <= 1024,
               "descriptor block");
 static_assert(NOALLOC_TABLE % NOALLOC_ALIGN == 0, "table alignment");
@@ -146,6 +150,11 @@ struct DevBuf {
       return fail(KMC_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
     }
     return KMC_OK;
+  }
+  void release() {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    n = cap = 0;
   }
   template <class T>
   T* as() const {
@@ -221,6 +230,10 @@ struct Engine {
   std::vector<int> eset_layout;
   DevBuf layouts_dev, esets_dev;
   DevBuf stage;   // staged energy sets of kmc_eset_write_many
+  // state records of the FP64 kernel's workgroups: every launch runs on `stream`
+  // and starts its records empty, so all of them share this one buffer (at most
+  // PLAIN_STATES_MAX bytes; freed by kmc_reset)
+  DevBuf plain_states;
   std::vector<Batch*> batches;
   bool layouts_dirty = true, esets_dirty = true;
   // bumped whenever layouts_dev or esets_dev moves to a new device address:
@@ -1144,14 +1157,21 @@ int launch_fp32(Batch* B, const kmc_run_opts& o, const std::vector<Fp32Launch>& 
   return KMC_OK;
 }
 
+// State records of the FP64 kernel: at most this much device memory for all
+// workgroups of a launch, and at most PLAIN_SLOTS_MAX per workgroup (one
+// trajectory at +-300 kT visits 500 to 2000 states in 2e4 hops).
+constexpr size_t PLAIN_STATES_MAX = (size_t)512 << 20;
+constexpr int PLAIN_SLOTS_MAX = 1024;
+
 // The FP64 dense kernel over ntraj trajectories (one wave each) whose layouts
 // have at most S sites and N acceptors: the layout's tables staged in LDS when
-// they fit.
-int launch_plain(PlainParams p, int S, int N, bool rec, int64_t ntraj, hipStream_t s) {
+// they fit.  `states` (nstates bytes): caller's memory for the state records,
+// or null for the engine's.
+int launch_plain(PlainParams p, int S, int N, bool rec, int64_t ntraj, hipStream_t s,
+                 int32_t* queue, void* states, size_t nstates) {
+  Engine& E = eng();
   const size_t cap = (size_t)160 * 1024;
-  const bool stage = plain_lds_bytes(S, N, true) <= cap;
-  const size_t lds = plain_lds_bytes(S, N, stage);
-  if (lds > cap) return fail(KMC_ERR_LIMIT, "FP64 kernel needs %zu bytes of LDS", lds);
+  const bool stage = plain_lds_bytes(S, N, 64, true) <= cap;
   using K = void (*)(PlainParams);
   K k = rec ? (stage ? (K)kmc_plain_fp64_kernel<true, true, false> : (K)kmc_plain_fp64_kernel<true, false, false>)
             : (stage ? (K)kmc_plain_fp64_kernel<false, true, false> : (K)kmc_plain_fp64_kernel<false, false, false>);
@@ -1159,9 +1179,44 @@ int launch_plain(PlainParams p, int S, int N, bool rec, int64_t ntraj, hipStream
     if (rec) return fail(KMC_ERR_UNSUPPORTED, "phase timing runs without records");
     k = stage ? (K)kmc_plain_fp64_kernel<false, true, true> : (K)kmc_plain_fp64_kernel<false, false, true>;
   }
+  p.smax = S;
+  p.nmax = N;
+  p.npairs = plain_pairs(S, N);
+  p.state_bytes = (int64_t)plain_state_bytes(S, N);
+  p.ntraj = (int32_t)ntraj;
+  // workgroups that fit on the GPU at once (one per CU at least) share the
+  // records' memory; the others' trajectories wait in the queue
+  int64_t grid = ntraj;
+  int slots = PLAIN_SLOTS_MAX;
+  if (ntraj > E.cu_count) {
+    slots = 64;
+    const size_t lds = plain_lds_bytes(S, N, slots, stage);
+    int per_cu = 0;
+    HIPOK(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    HIPOK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, 64, lds));
+    grid = std::min<int64_t>(ntraj, (int64_t)std::max(1, per_cu) * E.cu_count);
+  }
+  while (slots > 1 && plain_lds_bytes(S, N, slots, stage) > cap) slots /= 2;
+  const size_t most = states ? nstates : PLAIN_STATES_MAX;
+  while (slots > 1 && (size_t)grid * slots * p.state_bytes > most) slots /= 2;
+  if (!states) {
+    int st = KMC_OK;
+    while ((st = E.plain_states.alloc((size_t)grid * slots * p.state_bytes)) && slots > 1) slots /= 2;
+    if (st) return st;
+    states = E.plain_states.p;
+  }
+  p.states = static_cast<unsigned char*>(states);
+  p.slots = slots;
+  p.queue = grid < ntraj ? queue : nullptr;
+  const size_t lds = plain_lds_bytes(S, N, slots, stage);
+  if (lds > cap) return fail(KMC_ERR_LIMIT, "FP64 kernel needs %zu bytes of LDS", lds);
   HIPOK(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  if (p.queue) {
+    void* qa[] = {&p.queue};
+    HIPOK(hipLaunchKernel((const void*)kmc_queue_reset_kernel, dim3(1), dim3(1), qa, 0, s));
+  }
   void* args[] = {&p};
-  HIPOK(hipLaunchKernel((const void*)k, dim3((unsigned)ntraj), dim3(64), args, lds, s));
+  HIPOK(hipLaunchKernel((const void*)k, dim3((unsigned)grid), dim3(64), args, lds, s));
   return KMC_OK;
 }
 
@@ -1188,7 +1243,7 @@ int enqueue_fp64(Batch* B, const kmc_run_opts& o, hipStream_t s, const double* u
   p.occ_time = rec ? B->occ_time.as<double>() : nullptr;
   p.se_out = se_out;
   p.phases = phases;
-  return launch_plain(p, B->smax, B->nmax, rec, B->ntraj, s);
+  return launch_plain(p, B->smax, B->nmax, rec, B->ntraj, s, B->queue.as<int32_t>(), nullptr, 0);
 }
 
 int batch_run_locked(int32_t id, const kmc_run_opts* opts) {
@@ -1313,6 +1368,7 @@ int kmc_reset(void) {
   E.esets_host.clear();
   E.eset_layout.clear();
   E.layouts_dirty = E.esets_dirty = true;
+  E.plain_states.release();
   return KMC_OK;
 }
 
@@ -1909,7 +1965,7 @@ int kmc_simulate_discrete_noalloc(int64_t N, int64_t P, double nu, double kT, do
   p.traffic = (rec && traffic) ? dtr : nullptr;
   p.occ_time = rec ? dot : nullptr;
   p.se_out = dse;
-  if ((st = launch_plain(p, S, n, rec, 1, s))) return st;
+  if ((st = launch_plain(p, S, n, rec, 1, s, nullptr, base + NA_STATES, NOALLOC_STATES))) return st;
   TrajOut r;
   HIPOK(hipMemcpyAsync(&r, dO, sizeof r, hipMemcpyDeviceToHost, s));
   if (hops > 0 && N) HIPOK(hipMemcpyAsync(site_energies, dse, sizeof(double) * N, hipMemcpyDeviceToHost, s));

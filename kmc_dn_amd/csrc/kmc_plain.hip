@@ -16,40 +16,64 @@
 //     (:100-110); u == 0 selects k = 0 exactly as the reference's scan does.
 // This file is compiled with -ffp-contract=off: no a*b+c is fused.
 //
-// One wave (64 lanes) per trajectory.  The possible pairs of a hop have a
-// closed structure (_transition_possible, :137-163): rows of occupied acceptors
-// (ascending) hop into [empty acceptors ascending, then the electrodes], and
-// then each electrode row hops into the empty acceptors.  Two short LDS lists
-// (occupied acceptors; empty acceptors followed by electrodes) built with
-// ballots give every list position its (row, column) by one small division,
-// so the rates are lane-parallel over the compacted list.  Only the prefix
-// chain is serial: one lane runs it from registers, 8 values per LDS block in
-// two alternating register sets (the next block's loads in flight during the
-// current block's adds).  Uniforms and the clock's -log(1 - u) are computed
-// lane-parallel for 64 hops at a time.  The
-// event search is monotone (the prefix never decreases and the quotient by
-// the total is monotone), so two lane-parallel rounds find the first index
-// (a coarse pass over 64 block ends, then the block).  With STAGE the layout's
-// tables (1/d, tc, (I_0*R)/d) are copied to LDS once per trajectory.
+// One wave (64 lanes) per trajectory.  Three paths take a hop, all with the
+// same operations on the same values, so which of them took it changes no bit:
+//
+//  * An evaluated state: the rates of the possible pairs and their sequential
+//    prefix sum.  The possible pairs of a hop have a closed structure
+//    (_transition_possible, :137-163): rows of occupied acceptors (ascending)
+//    hop into [empty acceptors ascending, then the electrodes], and then each
+//    electrode row hops into the empty acceptors.  Two short LDS lists
+//    (occupied acceptors; empty acceptors followed by electrodes) built with
+//    ballots give every list position its (row, column) by one small division,
+//    so the rates are lane-parallel over the compacted list.  Only the prefix
+//    chain is serial: one lane runs it from registers, 8 values per LDS block
+//    in two alternating register sets (the next block's loads in flight during
+//    the current block's adds).  About 10,000 cycles at N = 30, P = 8.
+//  * A cached state.  Everything a hop needs of its state is a function of the
+//    occupation alone (the energies are summed afresh for every state), so the
+//    first visit stores it and every later one reads it: the quotients
+//    problist[k]/total of the kept entries, their events, 1/total.  The event
+//    is then one lane-parallel search, about 400 cycles.  Trajectories revisit
+//    a few states: of 2e4 hops at N = 30, P = 8 and 1 kT 0.1-0.3 % are first
+//    visits; at +-300 kT 2-10 % fall outside the last 1024 states (2-94 %
+//    outside the last two, which is why the cache holds many).  The records
+//    live in global memory (a state is up to 10 B per possible pair; the ones
+//    in use stay in the CU's L1 and the XCD's L2), their tags in LDS: sets of
+//    up to 64 ways, one tag per lane, so a lookup is one LDS read and a
+//    ballot.
+//  * A run of hops back and forth between two states (a leap).  Whether the hop
+//    with event uniform u leads from A to B depends on u alone: lo < u <= hi,
+//    the quotients around the event.  The lanes test the 64 hops of a uniform
+//    block at once; the run of hops that pass is applied together, its clock
+//    and occupation times added one by one in hop order as the reference adds
+//    them (about 20 cycles a hop).
+//
+// Uniforms and the clock's -log(1 - u) are computed lane-parallel for 64 hops
+// at a time.  With STAGE the layout's tables (1/d, tc, (I_0*R)/d) are copied to
+// LDS once per trajectory.  Workgroups take trajectories from a queue when the
+// batch has more of them than fit on the GPU at once; the state records belong
+// to the workgroup and start empty with every trajectory.
 #include "kmc_device.h"
 
 namespace kmc {
 
-// LDS carve-up for S sites, N acceptors (all offsets in doubles, 16-byte aligned).
+// LDS carve-up for layouts of at most S sites, N acceptors and npairs possible
+// pairs, and `slots` state records (all offsets in doubles, 16-byte aligned).
 struct PlainLds {
-  size_t se, buf, lists, invd, tc, ird, total;
-  __host__ __device__ PlainLds(int S, int N, bool stage) {
+  size_t se, buf, lists, invd, tc, ird, tags, next, total;
+  __host__ __device__ PlainLds(int S, int N, int npairs, int slots, bool stage) {
     auto up2 = [](size_t x) { return (x + 1) & ~(size_t)1; };
     const size_t SS = (size_t)S * S;
     se = 0;
     buf = up2(S);
-    // possible pairs: nA (N - nA + P) + P (N - nA) <= N^2/4 + P N for nA occupied
-    const size_t npairs = (size_t)N * N / 4 + (size_t)(S - N) * N + 16;
-    lists = buf + up2(npairs);   // int16: occupied acceptors [N], targets [S], kept [npairs]
+    lists = buf + up2(npairs + 16);   // int16: occupied acceptors [N], targets [S], kept [npairs]
     invd = lists + up2(((size_t)N + S + npairs + 3) / 4);
     tc = invd + (stage ? up2((size_t)N * N) : 0);
     ird = tc + (stage ? up2(SS) : 0);
-    total = ird + (stage ? up2(SS) : 0);
+    tags = ird + (stage ? up2(SS) : 0);
+    next = tags + 2 * (size_t)slots;   // two words per tag, then one int per set of 64 ways
+    total = next + up2(((size_t)slots + 127) / 128);
   }
 };
 
@@ -69,13 +93,27 @@ __device__ __forceinline__ int div_small(int x, int d, float rcp, int& r) {
   return q;
 }
 
+// A state's tag: the occupation (acceptors 0-63 in the first word, 64-79 in the
+// low bits of the second), bit 63 of the second word set, its kept entries
+// above bit 32.
+constexpr uint64_t TAG_VALID = 1ull << 63;
+constexpr uint64_t TAG_STATE = TAG_VALID | 0xFFFFull;
+
+// State records of one workgroup: {1/total, total}, then the quotients of the
+// kept entries, then their events (row << 8 | column).
+struct StateRecord {
+  double* head;
+  __device__ __forceinline__ double* quot() const { return head + 2; }
+  __device__ __forceinline__ uint16_t* event(int cap) const {
+    return reinterpret_cast<uint16_t*>(head + 2 + cap);
+  }
+};
+
 // PHASE: the phase-timing instantiation (shader-clock reads at the phase
 // boundaries of every hop; the work is unchanged).
 template <bool REC, bool STAGE, bool PHASE>
-__global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int t = blockIdx.x;
-  const int lane = threadIdx.x;
+__device__ __forceinline__ void plain_trajectory(const PlainParams& p, const int t, const int lane,
+                                 unsigned char* smem) {
   const TrajDev td = p.trajs[t];
   const LayoutDev L = p.layouts[td.layout];
   const EsetDev es = p.esets[td.eset];
@@ -87,7 +125,7 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
   const bool kT1 = kT == 1.0, nu1 = nu == 1.0;
 
   double* dl = reinterpret_cast<double*>(smem);
-  const PlainLds off(S, N, STAGE);
+  const PlainLds off(p.smax, p.nmax, p.npairs, p.slots, STAGE);
   double* se = dl + off.se;
   double* buf = dl + off.buf;     // rates of the possible pairs, then their prefix sums
   int16_t* srcA = reinterpret_cast<int16_t*>(dl + off.lists);   // occupied acceptors
@@ -109,8 +147,19 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
     tcp = b;
     irdp = c;
   }
+  // the state records' tags: sets of `ways` (a power of two, at most 64)
+  uint64_t* tags = reinterpret_cast<uint64_t*>(dl + off.tags);
+  int* next_way = reinterpret_cast<int*>(dl + off.next);
+  const int ways = min(p.slots, 64), sets = p.slots / ways;
+  for (int k = lane; k < p.slots; k += 64) tags[2 * k + 1] = 0;
+  for (int k = lane; k < sets; k += 64) next_way[k] = 0;
+  auto record = [&](int slot) {
+    return StateRecord{reinterpret_cast<double*>(
+        p.states + ((size_t)blockIdx.x * p.slots + slot) * p.state_bytes)};
+  };
 
-  Occ4 occ{td.occ[0], td.occ[1], td.occ[2], td.occ[3]};
+  // acceptors (N <= 80) live in the first two words
+  uint64_t occ0 = td.occ[0], occ1 = td.occ[1];
   // lanes of site chunk c (site lane + 64c) holding acceptors; S <= 80 < 128
   const uint64_t acc0 = N >= 64 ? ~0ull : ((1ull << N) - 1);
   const uint64_t acc1 = N <= 64 ? 0ull : ((1ull << (N - 64)) - 1);
@@ -124,8 +173,9 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
   double ot0 = 0.0, ot1 = 0.0;    // post-hop occupation time, sites lane and lane+64
   double time = 0.0;
   int32_t status = ST_OK;
-  const int64_t total_hops = td.prehops + td.hops;
-  int64_t h = 0;
+  // prehops + hops <= INT32_MAX is checked when a batch is created
+  const int prehops = (int)td.prehops, total_hops = (int)(td.prehops + td.hops);
+  int h = 0;
   uint64_t ph[PLAIN_PHASES] = {};
   uint64_t tp = PHASE ? __builtin_amdgcn_s_memtime() : 0;
   // cycles since the last mark into phase k
@@ -140,8 +190,8 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
   // and clock logarithms at a time, read with readlane per hop (the same
   // values and operations as per hop)
   double lg_lane = 0.0, ue_lane = 0.0;
-  auto refill = [&](int64_t hh) {
-    const int64_t hk = (hh & ~(int64_t)63) + lane;
+  auto refill = [&](int hh) {
+    const int64_t hk = (hh & ~63) + (int64_t)lane;
     double uc = 0.5, ue = 0.5;
     if (p.uniforms) {
       if (hk < total_hops) {
@@ -154,25 +204,16 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
     lg_lane = -log(1.0 - uc);
     ue_lane = ue;
   };
-  // every scalar load of the set-up has returned before the loop: LDS
-  // operations alone then complete in order, so the waits for the prefix
-  // chain's blocks count only the operations issued after each block
-  __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
-  for (; h < total_hops; ++h) {
-    const bool tally = h >= td.prehops;
-    if (h == td.prehops) {   // reset() between prehops and hops (:562-585)
-      time = 0.0;
-      eo = 0;
-      ot0 = ot1 = 0.0;
-    }
-    if ((h & 63) == 0) refill(h);
+
+  // The pair lists and site energies of occupation (q0, q1); sets nA, cE.
+  int nA = 0, cE = 0;
+  auto energies = [&](uint64_t q0, uint64_t q1) {
     // occupied / empty acceptors as wave-uniform masks of the two site chunks
-    const uint64_t o0 = occ.a & acc0, o1 = occ.b & acc1;
+    const uint64_t o0 = q0 & acc0, o1 = q1 & acc1;
     const uint64_t e0 = acc0 & ~o0, e1 = acc1 & ~o1;
     // the lists: occupied acceptors, then targets (empty acceptors, electrodes)
-    const int nA = __builtin_popcountll(o0) + __builtin_popcountll(o1);
-    const int cE = N - nA;
-    const int cA = cE + P;
+    nA = __builtin_popcountll(o0) + __builtin_popcountll(o1);
+    cE = N - nA;
     {
       const bool oc0 = (o0 >> lane) & 1ull, oc1 = (o1 >> lane) & 1ull;
       const bool em0 = (e0 >> lane) & 1ull, em1 = (e1 >> lane) & 1ull;
@@ -183,8 +224,6 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
       if (em1) tgt[lo_e + mbcnt(e1)] = (int16_t)(lane + 64);
       if (lane < P) tgt[cE + lane] = (int16_t)(N + lane);
     }
-    const int nAA = nA * cA;
-    const int n = nAA + P * cE;
     wave_lds_sync();
     mark(1);
     // site energies, :59-66: the empty acceptors j (tgt[0..cE), ascending),
@@ -216,6 +255,29 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
     }
     wave_lds_sync();
     mark(0);
+  };
+
+  // Evaluates occupation (occ0, occ1): leaves the kept entries' prefix sums in
+  // buf[0..ns) and their list positions in kidx, returns the total.
+  int ns = 0;                // entries kept (wave-uniform)
+  float rA = 0.f, rE = 0.f;
+  int cA = 0, nAA = 0;
+  auto pair_of = [&](int idx, int& i, int& j) {
+    int r;
+    if (idx < nAA) {
+      const int q = div_small(idx, cA, rA, r);
+      i = srcA[q];
+    } else {
+      const int q = div_small(idx - nAA, cE, rE, r);
+      i = N + q;
+    }
+    j = tgt[r];
+  };
+  auto evaluate = [&]() -> double {
+    energies(occ0, occ1);
+    cA = cE + P;
+    nAA = nA * cA;
+    const int n = nAA + P * cE;
     // rates of the possible pairs in row-major order, :69-87; two list entries
     // per lane and round, computed side by side (entries past n are evaluated
     // at n - 1 and dropped).
@@ -230,19 +292,8 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
     // entry, and the dropped entries' partial sums equal the kept entry's
     // before them.  The kept rates go to buf[0..ns) and their list positions
     // to kidx.
-    const float rA = cA > 0 ? __builtin_amdgcn_rcpf((float)cA) : 0.f;
-    const float rE = cE > 0 ? __builtin_amdgcn_rcpf((float)cE) : 0.f;
-    auto pair_of = [&](int idx, int& i, int& j) {
-      int r;
-      if (idx < nAA) {
-        const int q = div_small(idx, cA, rA, r);
-        i = srcA[q];
-      } else {
-        const int q = div_small(idx - nAA, cE, rE, r);
-        i = N + q;
-      }
-      j = tgt[r];
-    };
+    rA = cA > 0 ? __builtin_amdgcn_rcpf((float)cA) : 0.f;
+    rE = cE > 0 ? __builtin_amdgcn_rcpf((float)cE) : 0.f;
     auto rate_of = [&](int i, int j) {
       const int k = i * S + j;
       double dE;
@@ -254,7 +305,7 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
       return tcp[k] * m;
     };
     uint32_t hcarry = 0;   // running maximum of the high words (wave-uniform)
-    int ns = 0;            // entries kept so far (wave-uniform)
+    ns = 0;
     auto keep = [&](double r, int idx) {
       const bool valid = idx < n;
       const uint32_t hi = valid ? (uint32_t)((uint64_t)__double_as_longlong(r) >> 32) : 0u;
@@ -324,55 +375,234 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
         buf[idx] = acc;
       }
     }
-    const double total = readlane_f64(acc, 0);
-    mark(3);
-    if (p.totals && t == 0 && lane == 0) p.totals[h] = total;
-    if (total == 0.0) {   // reference: ZeroDivisionError at 1/problist[-1]
-      status = ST_ZERO_RATE;
-      break;
+    return readlane_f64(acc, 0);
+  };
+
+  // The way of the current state in its set (-1: not cached); sets `set`, `ns`.
+  int set = 0;
+  auto lookup = [&]() -> int {
+    // multiplicative mix of the occupation words (few sets: any spread will do)
+    uint32_t x = (uint32_t)occ0 * 0x9E3779B1u ^ (uint32_t)(occ0 >> 32) * 0x85EBCA77u ^
+                 (uint32_t)occ1 * 0xC2B2AE3Du;
+    x *= 0x27D4EB2Fu;
+    set = (int)(x >> 20) & (sets - 1);
+    const ulonglong2 tg =
+        *reinterpret_cast<const ulonglong2*>(tags + 2 * (set * ways + (lane & (ways - 1))));
+    const uint64_t m = ballot(tg.x == occ0 && (tg.y & TAG_STATE) == (occ1 | TAG_VALID));
+    if (!m) return -1;
+    const int way = __builtin_ctzll(m) & (ways - 1);
+    ns = (int)((uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(tg.y >> 32), way) & 0xFFFFu);
+    return way;
+  };
+
+  // The hop before the current one: where it started, its event and bounds.  A
+  // hop that undoes it makes (state before, current state) a pair, whose two
+  // events the leap tests.
+  struct Hop {
+    double lo, hi, scale, total;   // the event is taken iff lo < u <= hi
+    uint64_t s0, s1;               // occupation it starts from
+    int from, to;
+  };
+  Hop A{}, B{};        // A: from the current state to B's start; B: the way back
+  bool pair = false;   // A and B hold
+  bool prev = false;   // B holds the hop just taken
+  uint64_t last0 = occ0, last1 = occ1;   // occupation the last hop started from
+  // every scalar load of the set-up has returned before the loop: LDS
+  // operations alone then complete in order, so the waits for the prefix
+  // chain's blocks count only the operations issued after each block
+  __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
+  while (h < total_hops) {
+    const bool tally = h >= prehops;
+    if (h == prehops) {   // reset() between prehops and hops (:562-585)
+      time = 0.0;
+      eo = 0;
+      ot0 = ot1 = 0.0;
     }
-    const double lg = readlane_f64(lg_lane, (int)(h & 63));
-    const double ue = readlane_f64(ue_lane, (int)(h & 63));
-    const double scale = 1.0 / total;
-    const double hop_time = lg * scale;
-    wave_lds_sync();
-    mark(4);
+    const int hl = h & 63;
+    if (hl == 0) refill(h);
+    if (pair) {
+      // lane k (>= hl) starts its hop in A's state when k - hl is even
+      const bool inA = ((lane ^ hl) & 1) == 0;
+      const uint64_t ok = ballot(ue_lane > (inA ? A.lo : B.lo) && ue_lane <= (inA ? A.hi : B.hi));
+      const uint64_t no = ~(ok >> hl);
+      int n = no ? __builtin_ctzll(no) : 64;
+      n = min(n, min(64 - hl, (tally ? total_hops : prehops) - h));
+      if (n > 0) {
+        const double dts = lg_lane * (inA ? A.scale : B.scale);
+        if (t == 0 && lane >= hl && lane < hl + n) {
+          const int hk = (h & ~63) + lane;
+          if (p.events) p.events[hk] = inA ? A.from * S + A.to : B.from * S + B.to;
+          if (p.totals) p.totals[hk] = inA ? A.total : B.total;
+        }
+        // the clock and, post-hop (:126-130), the occupation times in hop order
+        if (REC && tally) {
+          const bool a0 = (A.s0 >> lane) & 1ull, b0 = (B.s0 >> lane) & 1ull;
+          const bool a1 = (A.s1 >> lane) & 1ull, b1 = (B.s1 >> lane) & 1ull;
+          for (int k = 0; k < n; ++k) {
+            const double d = readlane_f64(dts, hl + k);
+            time += d;
+            if ((k & 1) ? a0 : b0) ot0 += d;
+            if (N > 64) {
+              if ((k & 1) ? a1 : b1) ot1 += d;
+            }
+          }
+          if (p.traffic && lane == 0) {
+            double* tr = p.traffic + (size_t)t * SS;
+            unsafeAtomicAdd(tr + A.from * S + A.to, (double)((n + 1) >> 1));
+            if (n > 1) unsafeAtomicAdd(tr + B.from * S + B.to, (double)(n >> 1));
+          }
+        } else {
+          int k = 0;
+          for (; k + 4 <= n; k += 4) {
+            double d[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) d[q] = readlane_f64(dts, hl + k + q);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) time += d[q];
+          }
+          for (; k < n; ++k) time += readlane_f64(dts, hl + k);
+        }
+        const int e = N + lane;
+        const int dA = (lane < P && A.to == e ? 1 : 0) - (lane < P && A.from == e ? 1 : 0);
+        const int dB = (lane < P && B.to == e ? 1 : 0) - (lane < P && B.from == e ? 1 : 0);
+        eo += ((n + 1) >> 1) * dA + (n >> 1) * dB;
+        h += n;
+        last0 = (n & 1) ? A.s0 : B.s0;
+        last1 = (n & 1) ? A.s1 : B.s1;
+        if (n & 1) {
+          const Hop x = A;
+          A = B;
+          B = x;
+          occ0 = A.s0;
+          occ1 = A.s1;
+        }
+        mark(6);
+        continue;
+      }
+    }
+    // the state's record: read, or evaluated and stored first
+    int way = lookup();
+    if (way < 0) {
+      const double total = evaluate();
+      mark(3);
+      if (total == 0.0) {   // reference: ZeroDivisionError at 1/problist[-1]
+        if (p.totals && t == 0 && lane == 0) p.totals[h] = total;
+        status = ST_ZERO_RATE;
+        last0 = occ0;
+        last1 = occ1;
+        break;
+      }
+      way = __builtin_amdgcn_readfirstlane(next_way[set]);
+      if (lane == 0) {
+        next_way[set] = (way + 1) & (ways - 1);
+        tags[2 * (set * ways + way)] = occ0;
+        tags[2 * (set * ways + way) + 1] = occ1 | TAG_VALID | ((uint64_t)ns << 32);
+      }
+      const StateRecord r = record(set * ways + way);
+      double* q = r.quot();
+      uint16_t* ev = r.event(p.npairs);
+      for (int k = lane; k < ns; k += 64) {
+        int i, j;
+        pair_of(kidx[k], i, j);
+        q[k] = buf[k] / total;
+        ev[k] = (uint16_t)(i << 8 | j);
+      }
+      if (lane == 0) {
+        r.head[0] = 1.0 / total;
+        r.head[1] = total;
+      }
+      wave_lds_sync();   // this wave's later loads see the record (memory order within a wave)
+      mark(4);
+    }
     // first k with problist[k]/total >= u, :103-110 (monotone in k): a kept
     // entry, since a dropped one repeats the partial sum of the kept entry
-    // before it
-    int from = 0, to = 0;   // u == 0 and no match: the reference's event 0, (0, 0)
-    if (ue != 0.0) {
-      const int stride = (ns + 63) >> 6;
-      const int end = min(ns, (lane + 1) * stride) - 1;
-      const bool hit = lane * stride < ns && buf[end] / total >= ue;
-      const uint64_t mc = ballot(hit);
-      if (mc) {
-        const int base = __builtin_ctzll(mc) * stride;
-        const int pos = base + lane;
-        const uint64_t mf = ballot(lane < stride && pos < ns && buf[pos] / total >= ue);
-        pair_of(kidx[base + __builtin_ctzll(mf)], from, to);   // the block's last entry hits
+    // before it.  Up to 256 entries are read at once; longer records first
+    // find the chunk of 64 by its last entry.
+    const StateRecord r = record(set * ways + way);
+    const double* q = r.quot();
+    const uint16_t* ev = r.event(p.npairs);
+    const double scale = r.head[0], total = r.head[1];
+    const double ue = readlane_f64(ue_lane, hl);
+    double lo = 0.0, hi = 0.0;
+    int code = -1;
+    if (ns <= 256) {
+      double qv[4];
+      int cv[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        if (64 * m >= ns) break;
+        const int k = min(64 * m + lane, ns - 1);
+        qv[m] = q[k];
+        cv[m] = ev[k];
       }
-      // the same on every lane: keep the event and the occupation it updates
-      // on the scalar unit
-      from = __builtin_amdgcn_readfirstlane(from);
-      to = __builtin_amdgcn_readfirstlane(to);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        if (64 * m >= ns) break;
+        const uint64_t hit = ballot(qv[m] >= ue);
+        if (hit) {
+          const int l = __builtin_ctzll(hit);
+          hi = readlane_f64(qv[m], l);
+          if (l > 0) lo = readlane_f64(qv[m], l - 1);
+          code = __builtin_amdgcn_readlane(cv[m], l);
+          break;
+        }
+        lo = readlane_f64(qv[m], 63);
+      }
+    } else {
+      const int nch = (ns + 63) >> 6;
+      const double end = q[min(64 * lane + 63, ns - 1)];
+      const uint64_t mc = ballot(lane < nch && end >= ue);
+      if (mc) {
+        const int c = __builtin_ctzll(mc);
+        if (c > 0) lo = readlane_f64(end, c - 1);
+        const int k = min(64 * c + lane, ns - 1);
+        const double qv = q[k];
+        const int cv = ev[k];
+        const int l = __builtin_ctzll(ballot(qv >= ue));
+        hi = readlane_f64(qv, l);
+        if (l > 0) lo = readlane_f64(qv, l - 1);
+        code = __builtin_amdgcn_readlane(cv, l);
+      }
     }
-    const int k_ev = from * S + to;
+    // u == 0 and no match: the reference's event 0, (0, 0)
+    const bool first = ue == 0.0 || code < 0;
+    const int from = first ? 0 : code >> 8, to = first ? 0 : code & 255;
     mark(5);
-    if (p.events && t == 0 && lane == 0) p.events[h] = k_ev;
+    // the event and the clock, :100
+    const double lg = readlane_f64(lg_lane, hl);
+    const double hop_time = lg * scale;
+    if (t == 0 && lane == 0) {
+      if (p.events) p.events[h] = from * S + to;
+      if (p.totals) p.totals[h] = total;
+    }
     // perform hop, :116-123
-    if (from < N) occ.assign(from, false);
-    else if (lane == from - N) eo -= 1;
-    if (to < N) occ.assign(to, true);
-    else if (lane == to - N) eo += 1;
+    last0 = occ0;
+    last1 = occ1;
+    if (from < N) {
+      if (from < 64) occ0 &= ~(1ull << from);
+      else occ1 &= ~(1ull << (from - 64));
+    } else if (lane == from - N) {
+      eo -= 1;
+    }
+    if (to < N) {
+      if (to < 64) occ0 |= 1ull << to;
+      else occ1 |= 1ull << (to - 64);
+    } else if (lane == to - N) {
+      eo += 1;
+    }
     // record, :126-130
     if (REC && tally) {
-      if (p.traffic && lane == 0) p.traffic[(size_t)t * SS + k_ev] += 1.0;
-      if (lane < N && occ.test(lane)) ot0 += hop_time;
-      if (lane + 64 < N && occ.test(lane + 64)) ot1 += hop_time;
+      if (p.traffic && lane == 0) unsafeAtomicAdd(p.traffic + (size_t)t * SS + from * S + to, 1.0);
+      if ((occ0 >> lane) & 1ull) ot0 += hop_time;
+      if ((occ1 >> lane) & 1ull) ot1 += hop_time;
     }
     time += hop_time;
-    wave_lds_sync();
+    ++h;
+    // a hop back to where the one before it started: A that hop, B this one
+    pair = prev && !first && occ0 == B.s0 && occ1 == B.s1;
+    if (pair) A = B;
+    B = Hop{lo, hi, scale, total, last0, last1, from, to};
+    prev = !first;
     mark(6);
   }
   if (PHASE && p.phases && t == 0 && lane == 0)
@@ -380,20 +610,38 @@ __global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
   TrajOut* o = p.out + t;
   if (lane == 0) {
     o->time = time;
-    o->hops_done = h > td.prehops ? h - td.prehops : 0;
+    o->hops_done = h > prehops ? h - prehops : 0;
     o->status = status;
-    o->occ[0] = occ.a;
-    o->occ[1] = occ.b;
-    o->occ[2] = occ.c;
-    o->occ[3] = occ.d;
+    o->occ[0] = occ0;
+    o->occ[1] = occ1;
+    o->occ[2] = td.occ[2];
+    o->occ[3] = td.occ[3];
   }
   if (lane < L.P) o->eo[lane] = eo;
   if (REC && p.occ_time) {
     if (lane < N) p.occ_time[(size_t)t * NMAX + lane] = ot0;
     if (lane + 64 < N) p.occ_time[(size_t)t * NMAX + lane + 64] = ot1;
   }
-  if (p.se_out)
+  if (p.se_out && total_hops > 0) {   // the energies the last hop saw
+    energies(last0, last1);
     for (int i = lane; i < N; i += 64) p.se_out[(size_t)t * NMAX + i] = se[i];
+  }
+}
+
+template <bool REC, bool STAGE, bool PHASE>
+__global__ void __launch_bounds__(64) kmc_plain_fp64_kernel(PlainParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int lane = threadIdx.x;
+  int t = blockIdx.x;
+  for (;;) {
+    plain_trajectory<REC, STAGE, PHASE>(p, t, lane, smem);
+    if (!p.queue) break;
+    // (the queue counts from 0; the first gridDim.x trajectories are taken)
+    if (lane == 0) t = (int)gridDim.x + atomicAdd(p.queue, 1);
+    t = __builtin_amdgcn_readfirstlane(t);
+    if (t >= p.ntraj) break;
+    wave_lds_sync();
+  }
 }
 
 template __global__ void kmc_plain_fp64_kernel<false, false, false>(PlainParams);
@@ -403,9 +651,25 @@ template __global__ void kmc_plain_fp64_kernel<true, true, false>(PlainParams);
 template __global__ void kmc_plain_fp64_kernel<false, true, true>(PlainParams);
 template __global__ void kmc_plain_fp64_kernel<false, false, true>(PlainParams);
 
-// LDS bytes the kernel needs for S sites, N acceptors.
-size_t plain_lds_bytes(int S, int N, bool stage) {
-  return PlainLds(S, N, stage).total * sizeof(double);
+// Possible pairs of any occupation of a layout with at most S sites and N
+// acceptors: nA (cE + P) + P cE for nA occupied and cE = N - nA empty ones.
+int plain_pairs(int S, int N) {
+  int most = 0;
+  for (int n = 0; n <= N; ++n) {
+    const int P = S - n < PMAX ? S - n : PMAX;
+    most = most > n * n / 4 + P * n ? most : n * n / 4 + P * n;
+  }
+  return (most + 3) & ~3;
+}
+
+// LDS bytes the kernel needs for S sites, N acceptors and `slots` state records.
+size_t plain_lds_bytes(int S, int N, int slots, bool stage) {
+  return PlainLds(S, N, plain_pairs(S, N), slots, stage).total * sizeof(double);
+}
+
+// Bytes of one state record: 1/total and total, then 10 B per possible pair.
+size_t plain_state_bytes(int S, int N) {
+  return (16 + 10 * (size_t)plain_pairs(S, N) + 127) & ~(size_t)127;
 }
 
 }  // namespace kmc

@@ -169,11 +169,23 @@ struct PlainParams {
   double* se_out;           // [ntraj * NMAX] final site_energies[0:N], or null
   uint64_t* phases;         // [PLAIN_PHASES] shader cycles per hop phase of trajectory 0
                             // (the phase-timing instantiation only), or null
+  // The state records of the workgroups: `slots` (a power of two) of state_bytes
+  // each per workgroup; npairs bounds the possible pairs of every layout, smax
+  // and nmax their sites and acceptors.
+  unsigned char* states;
+  int64_t state_bytes;
+  int32_t slots;
+  int32_t npairs;
+  int32_t smax, nmax;
+  int32_t* queue;           // trajectories beyond the grid, zero before launch; null: none
+  int32_t ntraj;
+  int32_t pad;
 };
 
 // Hop phases of the FP64 dense kernel timed by its phase-timing instantiation:
-// energies, pair lists, rates, prefix chain, uniforms and clock, event search,
-// hop and records.
+// energies, pair lists, rates and prefix chain of new states, storing their
+// records, event search of cached states, hops, leaps and records (with
+// uniforms and clock).
 constexpr int PLAIN_PHASES = 7;
 
 // Status codes written per trajectory (also returned by the C-ABI).
