@@ -216,12 +216,10 @@ typedef struct kmc_run_opts {
                                  the duration of a launch (schedulers, watchdogs).
                                  0 = none.  Refused with team kernels.  No reference
                                  counterpart. */
-  int32_t state_store;        /* FP32 one-chunk solo kernels (S <= 64): LDS slots
-                                 per trajectory for states evicted from its two-state
-                                 cache, restored instead of re-evaluated when the
-                                 trajectory returns to them.  0 = as many (at most 4)
-                                 as fit without lowering the resident workgroups per
-                                 CU, -1 = none, 1..4 = at most that many.  Changes no
+  int32_t state_store;        /* FP32 one-chunk solo kernels (S <= 64): states a
+                                 trajectory keeps besides the last two, looked up
+                                 instead of evaluated again when it returns to them.
+                                 0 = up to 62, -1 = none, 1..4 = that many.  Changes no
                                  result, only the time per hop.  No reference
                                  counterpart (the Go library's occupation cache,
                                  simulation.go:254-296, keeps every state). */
@@ -379,12 +377,13 @@ int kmc_probe_fp64_phases(int32_t batch, uint64_t* cycles, int32_t n);
  * path, with every launch on its kernel's phase-timing instantiation
  * (shader-clock reads at the phase boundaries of every hop), and returns the
  * shader cycles of each trajectory's first wave summed over trajectories:
- * cycles[0..6] = uniforms and FP64 recomputes, a miss's state-cache lookup,
- * energy update, electrode terms, row sums and team reduction, a miss's FP64
- * prefix scan and cache insert, clock and event selection, partner selection,
- * hop (occupation and tallies), a hit's lookup and copy; cycles[7] = the
- * number of state-cache hits, cycles[8] = the number of hops whose partner
- * prefix came from the state's entry (n >= 9).
+ * cycles[0..6] = uniforms and FP64 recomputes; the energy update, electrode
+ * terms, row sums and team reduction of a new state (or its lookup); its FP64
+ * prefix scan and record; event selection; partner selection; the hop and the
+ * insertion of its transition; hops by kept transitions and leaps.  cycles[7] =
+ * the number of hops from a state that the hop before led back into, cycles[8] =
+ * those by a kept transition (steps that keep none: by a partner prefix formed
+ * before), n >= 9.
  * Solo launches need a table form and 4 waves per workgroup, team launches
  * teams of 4 on 2 or 3 site chunks; no records, graph or resume.  The clock
  * reads wait for outstanding loads, so the instrumented hops run slower than

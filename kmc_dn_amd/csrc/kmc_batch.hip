@@ -8,8 +8,7 @@
 namespace kmc {
 
 // Table policies: the workgroup's W waves run W trajectories of one layout and
-// share its tables in LDS.  Layout: the waves' state stores (W *
-// store_wave_bytes(p.store_slots)), the waves' electrode factors (W*2*PMAX
+// share its tables in LDS.  Layout: the waves' electrode factors (W*2*PMAX
 // floats), the electrode weights (elw_lds_floats), the pair table
 // (S*S + 64C float2) and, for BT, the c table (N*S + 64C floats).  PH: the
 // phase-timing instantiation (run_trajectory).
@@ -22,10 +21,9 @@ kmc_batch_fp32_kernel(BatchParams p) {
   // from them) in scalar registers with scalar branches
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int sb = store_wave_bytes(p.store_slots);
-  unsigned char* store = sb ? smem + wave * sb : nullptr;
-  float* evc = reinterpret_cast<float*>(smem + W * sb) + wave * 2 * PMAX;
-  float* elw = reinterpret_cast<float*>(smem + W * sb) + W * 2 * PMAX;
+  unsigned char* area = p.states + ((size_t)blockIdx.x * W + wave) * p.state_area;
+  float* evc = reinterpret_cast<float*>(smem) + wave * 2 * PMAX;
+  float* elw = reinterpret_cast<float*>(smem) + W * 2 * PMAX;
   __shared__ int s_group;
   __shared__ int s_layout;
   if (threadIdx.x == 0) s_layout = -1;
@@ -38,7 +36,7 @@ kmc_batch_fp32_kernel(BatchParams p) {
     const GroupDev gd = p.groups[g];
     const LayoutDev L = p.layouts[gd.layout];
     // a network of S <= 64 sites runs in one-chunk code (its tables laid out
-    // for one chunk): the bits of any chunk count, with the state store
+    // for one chunk): the bits of any chunk count
     const bool one = C > 1 && L.S <= 64;
     const int Ce = one ? 1 : C;
     float2* tab = reinterpret_cast<float2*>(elw + elw_lds_floats(L.P, Ce));
@@ -61,11 +59,11 @@ kmc_batch_fp32_kernel(BatchParams p) {
       if (one) {
         const TabPolicy<1, BT> pol = TabPolicy<1, BT>::make(tab, ctab, elw, evc, L.S, lane);
         run_trajectory<1, REC, TabPolicy<1, BT>, 1, PRIO, PH, false>(p, gd.first + wave, L, pol,
-                                                                     lane, Team<1, 1>{}, store);
+                                                                     lane, Team<1, 1>{}, area);
       } else {
         const TabPolicy<C, BT> pol = TabPolicy<C, BT>::make(tab, ctab, elw, evc, L.S, lane);
         run_trajectory<C, REC, TabPolicy<C, BT>, 1, PRIO, PH>(p, gd.first + wave, L, pol, lane,
-                                                              Team<1, C>{}, store);
+                                                              Team<1, C>{}, area);
       }
     }
   }
@@ -73,15 +71,13 @@ kmc_batch_fp32_kernel(BatchParams p) {
 
 // Positions policy: every wave pulls its own groups and keeps only its layout's
 // site coordinates in LDS (at most 64*C float4), so a workgroup mixes layouts.
-// The waves' state stores follow the coordinates (W * store_wave_bytes).
 template <int C, int W, bool REC>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(C == 1 ? 4 : 1)))
 kmc_batch_pos_kernel(BatchParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   float4* pos = reinterpret_cast<float4*>(smem) + wave * (64 * C);
-  const int sb = store_wave_bytes(p.store_slots);
-  unsigned char* store = sb ? smem + W * 64 * C * sizeof(float4) + wave * sb : nullptr;
+  unsigned char* area = p.states + ((size_t)blockIdx.x * W + wave) * p.state_area;
   for (;;) {
     int g = 0;
     if (lane == 0) g = atomicAdd(p.queue, 1);
@@ -92,19 +88,19 @@ kmc_batch_pos_kernel(BatchParams p) {
     for (int k = lane; k < L.S; k += 64) pos[k] = L.pos4[k];
     wave_lds_sync();
     if (C > 1 && L.S <= 64) {
-      // a one-chunk network: the one-chunk code (fast hops and leaps, fewer
-      // instructions per hop); its trajectories' bits are those of any chunk count
+      // a one-chunk network: the one-chunk code (fewer instructions
+      // per hop); its trajectories' bits are those of any chunk count
       PosPolicy<1> pol;
       pol.init(pos, L, lane);
       for (int i = 0; i < gd.count; ++i)
         run_trajectory<1, REC, PosPolicy<1>, 1, true, false, false>(p, gd.first + i, L, pol, lane,
-                                                                    Team<1, 1>{}, store);
+                                                                    Team<1, 1>{}, area);
     } else {
       PosPolicy<C> pol;
       pol.init(pos, L, lane);
       for (int i = 0; i < gd.count; ++i)
         run_trajectory<C, REC, PosPolicy<C>, 1, true>(p, gd.first + i, L, pol, lane,
-                                                      Team<1, C>{}, store);
+                                                      Team<1, C>{}, area);
     }
     wave_lds_sync();
   }
@@ -167,9 +163,5 @@ size_t batch_lds_bytes(bool bt, int C, int W, int S, int N, int P) {
 }
 
 size_t pos_lds_bytes(int C, int W) { return (size_t)W * 64 * C * sizeof(float4); }
-
-// LDS bytes of the W waves' state stores of `slots` slots each (they come before
-// the table kernels' other LDS and after the positions kernels' coordinates).
-size_t store_lds_bytes(int W, int slots) { return (size_t)W * store_wave_bytes(slots); }
 
 }  // namespace kmc

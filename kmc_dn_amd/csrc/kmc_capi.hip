@@ -37,10 +37,12 @@ size_t plain_state_bytes(int S, int N);
 int plain_pairs(int S, int N);
 size_t batch_lds_bytes(bool bt, int C, int W, int S, int N, int P);
 size_t pos_lds_bytes(int C, int W);
-size_t store_lds_bytes(int W, int slots);
 template <int C, int T, bool REC, int FORM, bool PH>
 __global__ void kmc_team_kernel(BatchParams);
 size_t team_lds_bytes(int form, int C, int T, int S, int N, int P);
+template <int C, bool REC, int FORM>
+__global__ void kmc_split_kernel(BatchParams);
+size_t split_lds_bytes(int form, int C, int S, int N, int P);
 template <int C>
 __global__ void kmc_meanfield_kernel(MeanfieldParams);
 template <int C>
@@ -199,6 +201,7 @@ struct Batch {
     DevBuf groups;
     int32_t ngroups = 0;
     int smax = 0, nmax = 0, pmax = 0;
+    bool split = false;   // one trajectory per group, for the kernels that split by site chunks
   };
   Sub subs[KMC_MAX_BUCKETS];
   bool subs_built = false;
@@ -234,6 +237,10 @@ struct Engine {
   // and starts its records empty, so all of them share this one buffer (at most
   // PLAIN_STATES_MAX bytes; freed by kmc_reset)
   DevBuf plain_states;
+  // state records of the FP32 kernels' resident waves (32 KiB per wave and site
+  // chunk, at most 16 waves of one chunk or 12 of three per CU: 300 MB a launch;
+  // freed by kmc_reset)
+  DevBuf states;
   std::vector<Batch*> batches;
   bool layouts_dirty = true, esets_dirty = true;
   // bumped whenever layouts_dev or esets_dev moves to a new device address:
@@ -876,6 +883,34 @@ BatchKernel pick_pos_kernel(int C, int W, bool rec) {
   return nullptr;
 }
 
+BatchKernel pick_split_kernel(int C, bool rec, int form) {
+#define KMC_PICK(CC, FF)                                                     \
+  if (C == CC && form == FF)                                                 \
+    return rec ? (BatchKernel)kmc_split_kernel<CC, true, FF>                 \
+               : (BatchKernel)kmc_split_kernel<CC, false, FF>;
+  KMC_PICK(2, 1) KMC_PICK(2, 2) KMC_PICK(2, 3) KMC_PICK(3, 1) KMC_PICK(3, 2) KMC_PICK(3, 3)
+#undef KMC_PICK
+  return nullptr;
+}
+
+// Whether a solo launch over `ntraj` trajectories of layouts with at most S, N
+// and P sites gives each of them a wave per site chunk (kmc_split_kernel, the
+// same bits): while all of those waves fit beside each other, two on a SIMD (their
+// registers' limit; table forms: a workgroup on a CU, their LDS's).  10,000 hops,
+// ms solo / split: S = 148 in the positions form, 64 trajectories 30.7 / 13.7, 512
+// 47.1 / 21.1, 680 47.2 / 29.3 (1024 do not fit); S = 78, 64 of them 1.70 / 1.55, 1024
+// 6.79 / 6.11; S = 109 in table form 2, 256 of them 10.3 / 9.8, all states new 23.1 /
+// 20.5.
+constexpr int SPLIT_WAVES_PER_CU = 8;
+bool split_fits(int64_t ntraj, int form, int smax, int nmax, int pmax) {
+  const int C = (smax + 63) / 64;
+  if (C < 2) return false;
+  if (form != 3 && (ntraj > eng().cu_count ||
+                    split_lds_bytes(form, C, smax, nmax, pmax) > (size_t)160 * 1024))
+    return false;
+  return ntraj * C <= SPLIT_WAVES_PER_CU * (int64_t)eng().cu_count;
+}
+
 struct Fp32Launch {
   BatchKernel k = nullptr;
   int grid = 0, block = 0;
@@ -888,7 +923,7 @@ struct Fp32Launch {
 // phases: run the phase-timing instantiation, summing into phases[FP32_PHASES].
 int setup_launch(Batch* B, const kmc_run_opts& o, int form, int W, int team, int smax, int nmax,
                  int pmax, const DevBuf& groups, int32_t ngroups, int32_t* queue, int grid_cap,
-                 Fp32Launch& L, uint64_t* phases) {
+                 Fp32Launch& L, uint64_t* phases, bool split) {
   Engine& E = eng();
   const int C = (smax + 63) / 64;
   // recording kernels: occupation time (bit 0) and traffic (bit 1); the others
@@ -901,6 +936,10 @@ int setup_launch(Batch* B, const kmc_run_opts& o, int form, int W, int team, int
     k = pick_team_kernel(C, team, rec, form);
     lds = team_lds_bytes(form, C, team, smax, nmax, pmax);
     W = team;   // block of 64 * team threads, one trajectory per workgroup
+  } else if (split) {
+    k = pick_split_kernel(C, rec, form);
+    lds = split_lds_bytes(form, C, smax, nmax, pmax);
+    W = C;
   } else if (form == 3) {
     k = pick_pos_kernel(C, W, rec);
     lds = pos_lds_bytes(C, W);
@@ -924,35 +963,10 @@ int setup_launch(Batch* B, const kmc_run_opts& o, int form, int W, int team, int
   int per_cu = 0;
   HIPOK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, 64 * W, lds));
   if (per_cu <= 0) return fail(KMC_ERR_LIMIT, "kernel does not fit on a CU (LDS %zu)", lds);
-  // The state stores of one-chunk solo kernels: as many slots as leave the
-  // resident workgroups per CU unchanged.  They change no result.  (Kernels
-  // over several site chunks run their S <= 64 networks in one-chunk code
-  // without a store: their LDS would take room that a plan's team
-  // workgroups, placed beside them, need.)
-  int slots = 0;
-  if (team <= 1 && C == 1 && o.state_store >= 0) {
-    const int want = o.state_store > 0 ? std::min(o.state_store, STORE_MAX_SLOTS) : STORE_MAX_SLOTS;
-    for (int v = want; v > 0 && !slots; --v) {
-      const size_t l2 = lds + store_lds_bytes(W, v);
-      if (l2 > lds_cap) continue;
-      // (refused when l2 and the kernel's static LDS exceed a workgroup's share)
-      if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l2) !=
-          hipSuccess) {
-        (void)hipGetLastError();
-        continue;
-      }
-      int pc = 0;
-      HIPOK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc, (const void*)k, 64 * W, l2));
-      if (pc >= per_cu) {
-        slots = v;
-        lds = l2;
-      }
-    }
-  }
   // The graded issue priority of the hop pays while every group is resident at
   // once (4096 trajectories: +12 %); with groups queued behind full SIMDs the
   // variant without it is 2 % faster (65,536-trajectory IV sweep).
-  if (team <= 1 && form != 3 && !rec && !phases && ngroups > per_cu * E.cu_count) {
+  if (team <= 1 && !split && form != 3 && !rec && !phases && ngroups > per_cu * E.cu_count) {
     k = pick_batch_kernel(C, W, rec, form == 1, false);
     HIPOK(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     HIPOK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, 64 * W, lds));
@@ -960,7 +974,7 @@ int setup_launch(Batch* B, const kmc_run_opts& o, int form, int W, int team, int
   }
   int grid = per_cu * E.cu_count;
   if (grid_cap > 0) grid = std::min(grid, grid_cap);
-  const int work_units = (form == 3 && team <= 1) ? (ngroups + W - 1) / W : ngroups;
+  const int work_units = (form == 3 && team <= 1 && !split) ? (ngroups + W - 1) / W : ngroups;
   grid = std::max(1, std::min(grid, work_units));
   BatchParams& p = L.p;
   p.trajs = B->trajs.as<TrajDev>();
@@ -978,7 +992,9 @@ int setup_launch(Batch* B, const kmc_run_opts& o, int form, int W, int team, int
   p.resume = o.resume ? 1 : 0;
   p.phases = phases;
   p.time_limit = o.time_limit_us > 0 ? (int64_t)o.time_limit_us * E.wall_khz / 1000 : 0;
-  p.store_slots = slots;
+  // a positive state_store: the two last states and that many more
+  p.state_slots = o.state_store == 0 ? STATE_SLOTS : 2 + std::max(0, o.state_store);
+  p.state_area = (int64_t)C * STATE_SLOTS * STATE_RECORD_BYTES;
   L.k = k;
   L.grid = grid;
   L.block = 64 * W;
@@ -1010,11 +1026,25 @@ int build_bucket_groups(Batch* B) {
   Engine& E = eng();
   const int nb = (int)B->plan.size();
   std::vector<std::vector<GroupDev>> g(nb);
+  std::vector<int64_t> count(nb, 0);
   for (int b = 0; b < nb; ++b) B->subs[b].smax = B->subs[b].nmax = B->subs[b].pmax = 0;
   auto bucket_at = [&](int64_t k) {
     const TrajDev& t = B->host[k];
     return bucket_of(B, E.layouts[t.layout]->S, t.prehops + t.hops);
   };
+  for (int64_t k = 0; k < B->ntraj; ++k) {
+    const Layout* Ly = E.layouts[B->host[k].layout];
+    const int b = bucket_at(k);
+    if (b < 0) continue;   // (refused below)
+    ++count[b];
+    B->subs[b].smax = std::max(B->subs[b].smax, Ly->S);
+    B->subs[b].nmax = std::max(B->subs[b].nmax, Ly->N);
+    B->subs[b].pmax = std::max(B->subs[b].pmax, Ly->P);
+  }
+  for (int b = 0; b < nb; ++b)
+    B->subs[b].split = B->plan[b].team <= 1 && B->plan[b].grid <= 0 &&
+                       split_fits(count[b], B->plan[b].table_form, B->subs[b].smax,
+                                  B->subs[b].nmax, B->subs[b].pmax);
   int64_t i = 0;
   while (i < B->ntraj) {
     const Layout* Ly = E.layouts[B->host[i].layout];
@@ -1024,7 +1054,8 @@ int build_bucket_groups(Batch* B) {
                   B->host[i].layout, Ly->S,
                   (long long)(B->host[i].prehops + B->host[i].hops));
     const kmc_bucket& pb = B->plan[b];
-    const int W = (pb.table_form == 3 || pb.team > 1) ? 1 : pb.waves_per_group;
+    const int W =
+        (pb.table_form == 3 || pb.team > 1 || B->subs[b].split) ? 1 : pb.waves_per_group;
     int64_t j = i;
     while (j < B->ntraj && j - i < W && B->host[j].layout == B->host[i].layout && bucket_at(j) == b)
       ++j;
@@ -1034,9 +1065,6 @@ int build_bucket_groups(Batch* B) {
     gd.count = (int32_t)(j - i);
     gd.pad = 0;
     g[b].push_back(gd);
-    B->subs[b].smax = std::max(B->subs[b].smax, Ly->S);
-    B->subs[b].nmax = std::max(B->subs[b].nmax, Ly->N);
-    B->subs[b].pmax = std::max(B->subs[b].pmax, Ly->P);
     i = j;
   }
   for (int b = 0; b < nb; ++b) {
@@ -1050,6 +1078,25 @@ int build_bucket_groups(Batch* B) {
     if (st) return st;
   }
   B->subs_built = true;
+  return KMC_OK;
+}
+
+// The launches' state records in the engine's buffer: every run of every batch is
+// ordered on the engine stream, and the launches of one run have areas of
+// their own.  A captured graph holds the addresses: reg_gen tells it when they move.
+int place_states(std::vector<Fp32Launch>& Ls) {
+  Engine& E = eng();
+  size_t need = 0;
+  for (const Fp32Launch& L : Ls) need += (size_t)L.grid * (L.block / 64) * L.p.state_area;
+  const void* was = E.states.p;
+  int st = E.states.alloc(need);
+  if (E.states.p != was) ++E.reg_gen;
+  if (st) return st;
+  unsigned char* at = E.states.as<unsigned char>();
+  for (Fp32Launch& L : Ls) {
+    L.p.states = at;
+    at += (size_t)L.grid * (L.block / 64) * L.p.state_area;
+  }
   return KMC_OK;
 }
 
@@ -1070,11 +1117,11 @@ int prepare_fp32(Batch* B, const kmc_run_opts& o, std::vector<Fp32Launch>& out,
       Fp32Launch L;
       st = setup_launch(B, o, pb.table_form, pb.waves_per_group, pb.team, sb.smax, sb.nmax,
                         sb.pmax, sb.groups, sb.ngroups, q + 16 * b, pb.grid > 0 ? pb.grid : o.grid_limit, L,
-                        phases);
+                        phases, sb.split && !phases && o.grid_limit <= 0);
       if (st) return st;
       out.push_back(L);
     }
-    return KMC_OK;
+    return place_states(out);
   }
   const int C = (B->smax + 63) / 64;
   int form = o.table_form;
@@ -1087,14 +1134,16 @@ int prepare_fp32(Batch* B, const kmc_run_opts& o, std::vector<Fp32Launch>& out,
   const int team = o.team <= 1 ? 1 : o.team;
   if (team != 1 && team != 2 && team != 4) return fail(KMC_ERR_ARGS, "team must be 1, 2 or 4");
   if (form == 3 && (st = check_positions(B, -1))) return st;
-  // positions and teams: one trajectory per group
-  if ((st = build_groups(B, (form == 3 || team > 1) ? 1 : W))) return st;
+  const bool split = team <= 1 && !phases && o.grid_limit <= 0 &&
+                     split_fits(B->ntraj, form, B->smax, B->nmax, B->pmax);
+  // positions, teams and splits: one trajectory per group
+  if ((st = build_groups(B, (form == 3 || team > 1 || split) ? 1 : W))) return st;
   Fp32Launch L;
   if ((st = setup_launch(B, o, form, W, team, B->smax, B->nmax, B->pmax, B->groups, B->ngroups, q,
-                         o.grid_limit, L, phases)))
+                         o.grid_limit, L, phases, split)))
     return st;
   out.push_back(L);
-  return KMC_OK;
+  return place_states(out);
 }
 
 int launch_one(const Fp32Launch& L, hipStream_t s) {
@@ -1369,6 +1418,8 @@ int kmc_reset(void) {
   E.eset_layout.clear();
   E.layouts_dirty = E.esets_dirty = true;
   E.plain_states.release();
+  E.states.release();
+  ++E.reg_gen;
   return KMC_OK;
 }
 

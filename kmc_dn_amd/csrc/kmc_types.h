@@ -126,34 +126,29 @@ struct BatchParams {
                                 // instantiations only), or null
   int64_t time_limit;           // constant-rate clock ticks a solo trajectory runs before
                                 // it stops at its next recompute point; 0: none
-  int32_t store_slots;          // slots of each wave's LDS state store (one-chunk solo
-                                // trajectories; 0: none)
+  int32_t state_slots;          // states a one-chunk solo trajectory keeps, 2..STATE_SLOTS
+                                // (the others: STATE_SLOTS)
   int32_t pad2;
+  unsigned char* states;        // the waves' state records, state_area bytes per wave
+  int64_t state_area;
 };
 
-// The state store of a one-chunk solo trajectory: states evicted from its two
-// register entries, kept in LDS per wave.  Layout: STORE_MAX_SLOTS occupation
-// keys (u64), then STORE_MAX_SLOTS nonzero-row lane masks (u64), then per slot
-// the FP64 inclusive and exclusive row prefixes and the energies (FP32 values
-// held as FP64, so that every array of a slot has the same per-lane stride) of
-// the 64 lanes.
-constexpr int STORE_MAX_SLOTS = 4;
-constexpr int STORE_HEADER_BYTES = 2 * STORE_MAX_SLOTS * 8;
-constexpr int STORE_SLOT_BYTES = 64 * (8 + 8 + 8);
-constexpr int store_wave_bytes(int slots) {
-  return slots > 0 ? STORE_HEADER_BYTES + slots * STORE_SLOT_BYTES : 0;
-}
+// States a wave of the FP32 kernels keeps (one per lane), and the bytes of one's
+// record per site chunk: the FP32 row sums and energies of the 64 lanes.
+constexpr int STATE_SLOTS = 64;
+constexpr int STATE_RECORD_BYTES = 64 * (4 + 4);
+constexpr int STORE_MAX_SLOTS = 4;   // largest kmc_run_opts.state_store
 
 // Hop phases of the FP32 batched kernels timed by their phase-timing
 // instantiations (shader cycles of each trajectory's first wave, summed over
-// trajectories): 0 uniforms and FP64 recomputes (and fast-hop attempts that
-// fell through to the general step), 1 energy update, electrode terms, row
-// sums and team reduction of a miss, 2 FP64 prefix scan and cache insert of a
-// miss, 3 clock and event selection, 4 partner selection, 5 hop (occupation,
-// tallies) of the general step, 6 fast hops and leaps; slot 7 counts the hops
-// from a cached state, slot 8 those whose partner prefix came from the state's
-// entry, slot 9 those taken by leaps, slot 10 the new states restored from the
-// LDS state store instead of evaluated.
+// trajectories): 0 uniforms and FP64 recomputes, 1 energy update, electrode
+// terms, row sums and team reduction of a new state (or its lookup), 2 its FP64
+// prefix scan and record, 3 event selection of a new transition, 4 its partner
+// selection, 5 its insertion and the hop, 6 hops by kept transitions and leaps
+// (general steps: 0 to 5); slot 7 counts the
+// hops from a state that the hop before led back into, slot 8 those by a kept
+// transition (general steps: by a partner prefix formed before), slot 9 those taken by leaps, slot 10 the states found among the
+// kept ones instead of evaluated.
 constexpr int FP32_PHASES = 11;
 
 struct PlainParams {
