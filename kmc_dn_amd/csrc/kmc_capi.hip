@@ -43,8 +43,10 @@ size_t team_lds_bytes(int form, int C, int T, int S, int N, int P);
 template <int C, bool REC, int FORM>
 __global__ void kmc_split_kernel(BatchParams);
 size_t split_lds_bytes(int form, int C, int S, int N, int P);
-template <int C>
+template <int C, int Q, int W>
 __global__ void kmc_meanfield_kernel(MeanfieldParams);
+template <int C>
+__global__ void kmc_meanfield_tiled_kernel(MeanfieldParams);
 template <int C>
 __global__ void kmc_avg_current_kernel(MeanfieldParams);
 
@@ -166,6 +168,7 @@ struct DevBuf {
 
 struct Layout {
   int N = 0, P = 0, S = 0;
+  bool symmetric = true;            // transitions and acceptors' distances, to the bit
   std::vector<DevBuf*> eset_bufs;   // energy-set buffers created on this layout
   std::vector<int> eset_live;       // live energy sets per buffer
   std::vector<int32_t> eset_ids;    // energy-set id -> (position here)
@@ -388,6 +391,10 @@ int layout_create_locked(int64_t N, int64_t P, double nu, double kT, double I_0,
   L->N = n;
   L->P = (int)P;
   L->S = S;
+  for (int i = 0; i < S; ++i)
+    for (int j = 0; j < i; ++j)
+      L->symmetric = L->symmetric && tc[i * S + j] == tc[j * S + i] &&
+                     (i >= n || d[i * S + j] == d[j * S + i]);
   int st;
   if ((st = upload(L->tab32, tab)) || (st = upload(L->tabB, tabB)) || (st = upload(L->ccol, ccol)) ||
       (st = upload(L->elw, elw)) ||
@@ -1720,7 +1727,7 @@ int kmc_batch_destroy(int32_t batch) {
 
 namespace {
 
-// One wave per network; n networks of layouts[i] / esets[i].  avg_current: the
+// One workgroup per network; n networks of layouts[i] / esets[i].  avg_current: the
 // calcAverageCurrent evaluation (currents into eo_out), else probSimulate for
 // `steps` steps (occupation in/out).
 int meanfield_locked(bool avg_current, int32_t n, const int32_t* layouts, const int32_t* esets,
@@ -1734,6 +1741,7 @@ int meanfield_locked(bool avg_current, int32_t n, const int32_t* layouts, const 
   if (steps < 0) return fail(KMC_ERR_ARGS, "steps must be >= 0");
   if (n == 0) return KMC_OK;
   int smax = 0;
+  bool symmetric = true;
   for (int32_t i = 0; i < n; ++i) {
     const int32_t l = layouts[i], e = esets[i];
     if (l < 0 || l >= (int)E.layouts.size() || !E.layouts[l])
@@ -1741,6 +1749,7 @@ int meanfield_locked(bool avg_current, int32_t n, const int32_t* layouts, const 
     if (e < 0 || e >= (int)E.eset_layout.size() || E.eset_layout[e] != l)
       return fail(KMC_ERR_ARGS, "network %d: energy set %d does not belong to layout %d", i, e, l);
     smax = std::max(smax, E.layouts[l]->S);
+    symmetric = symmetric && E.layouts[l]->symmetric;
   }
   if ((st = sync_registry())) return st;
   const int C = (smax + 63) / 64;
@@ -1775,11 +1784,26 @@ int meanfield_locked(bool avg_current, int32_t n, const int32_t* layouts, const 
   mp.n = n;
   using K = void (*)(MeanfieldParams);
   K k = nullptr;
-  if (avg_current)
+  int block = 64;
+  size_t lds = 0;
+  if (avg_current) {
     k = C == 1 ? (K)kmc_avg_current_kernel<1> : C == 2 ? (K)kmc_avg_current_kernel<2> : (K)kmc_avg_current_kernel<3>;
-  else
-    k = C == 1 ? (K)kmc_meanfield_kernel<1> : C == 2 ? (K)kmc_meanfield_kernel<2> : (K)kmc_meanfield_kernel<3>;
-  hipLaunchKernelGGL(k, dim3(n), dim3(64), 0, E.stream, mp);
+  } else if (smax <= MF_LDS_SITES && symmetric) {
+    // pairs S (S + 1) / 2 over 512 threads of up to 5 (S = 64: 2080; two such
+    // workgroups fit a CU), 1024 of up to 6 (S = 110: 6105) or of up to 10 (S = 139: 9730)
+    mp.ld = mf_row(smax);
+    lds = (size_t)smax * mp.ld * sizeof(double);
+    k = smax <= 64 ? (K)kmc_meanfield_kernel<1, 5, 8>
+        : smax <= 110 ? (K)kmc_meanfield_kernel<2, 6, 16> : (K)kmc_meanfield_kernel<3, 10, 16>;
+    block = smax <= 64 ? 512 : 1024;
+  } else {
+    lds = (size_t)2 * MF_TILE * (64 * C + 1) * sizeof(double);
+    k = C == 1 ? (K)kmc_meanfield_tiled_kernel<1>
+        : C == 2 ? (K)kmc_meanfield_tiled_kernel<2> : (K)kmc_meanfield_tiled_kernel<3>;
+    block = 1024;
+  }
+  if (lds) HIPOK(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(k, dim3(n), dim3(block), lds, E.stream, mp);
   HIPOK(hipGetLastError());
   if (!avg_current) {
     HIPOK(hipMemcpyAsync(occupation, occ.p, na * sizeof(double), hipMemcpyDeviceToHost, E.stream));

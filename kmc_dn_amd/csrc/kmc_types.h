@@ -62,7 +62,7 @@ struct EsetDev {
 
 // Mean-field estimators of the Go library: probSimulate
 // (goSimulation/probabilitySimulation.go:53-157) and calcAverageCurrent
-// (goSimulation/simulation.go:671-736), one wave per network.
+// (goSimulation/simulation.go:671-736, one wave per network).
 struct MeanfieldParams {
   const LayoutDev* layouts;
   const EsetDev* esets;
@@ -77,8 +77,15 @@ struct MeanfieldParams {
   int64_t tstride;
   int64_t steps;
   int32_t n;
-  int32_t pad;
+  int32_t ld;                 // row length of the LDS pair table (kmc_meanfield_kernel)
 };
+
+// The LDS pair table of probSimulate: S rows of S | 1 doubles, 151 KiB at most (beside
+// 8 KiB of the sites' own).
+constexpr int MF_LDS_SITES = 139;
+constexpr int mf_row(int S) { return S | 1; }
+// the tiled kernel's two tiles of MF_TILE rows of 64 C + 1
+constexpr int MF_TILE = 32;
 
 struct TrajDev {
   int32_t layout;

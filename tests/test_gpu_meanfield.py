@@ -174,3 +174,48 @@ def test_kmc_class_estimators(gpu_engine):
     print("[gpu] kmc_dn.go_simulation(wrapperSimulateCombined)", flush=True)
     k.go_simulation(hops=5000, goSpecificFunction="wrapperSimulateCombined")
     assert k.time > 0 and np.isfinite(k.estimator.electrode_occupation).all()
+
+
+@pytest.mark.parametrize("N,P", [(1, 0), (1, 1), (2, 0), (31, 1), (56, 8), (57, 8), (102, 8), (103, 8), (131, 8),
+                                 (132, 8), (133, 8), (180, 12)])
+def test_pair_table_and_tiles_give_the_same_bits(gpu_engine, N, P):
+    """Sizes beside the pair table's variants (S = 64, 110, 139) and the largest: alone, in one
+    call with a network of 141 sites, whose table does not fit in LDS, and, up to rounding,
+    with transitions that are not symmetric to the last bit."""
+    steps, S = 40, N + P
+    net, big = random_network(7, N, P, M=0 if N < 4 else None, I_0=20.0, a=0.3), random_network(8, 133, 8, I_0=20.0, a=0.3)
+    print(f"[gpu] meanfield S={S}", flush=True)
+    (lay, es), (lb, eb) = _layout(net), _layout(big)
+    skew = dict(net, transitions_constant=net["transitions_constant"].copy())
+    skew["transitions_constant"][np.triu_indices(S, 1)] *= 1 + 3e-13
+    ls, e_skew = _layout(skew)
+    try:
+        occ0 = np.full((2, _lib.NMAX), 0.5)
+        occ0[0, :N] = np.linspace(0.2, 0.9, N)
+        for record in (False, True):
+            one = engine.meanfield_simulate([lay], es, steps, occ0[:1], record=record)
+            two = engine.meanfield_simulate([lay, lb], [es[0], eb[0]], steps, occ0, record=record)
+            ref = _oracle(net, steps, occ0[0, :N].copy(), record)
+            fields = ["occupation", "electrode_occupation", "site_energies", "time"]
+            for f in fields + (["average_occupation"] if record else []):
+                # (the entries past the network's sites are unspecified)
+                n = 1 if f == "time" else P if f == "electrode_occupation" else N
+                assert np.array_equal(np.atleast_1d(getattr(one, f)[0])[:n], np.atleast_1d(getattr(two, f)[0])[:n],
+                                      equal_nan=True), (f, record)
+            if record:
+                assert np.array_equal(one.traffic[0].ravel(), two.traffic[0].ravel()[:S * S], equal_nan=True)
+            if S == 1:
+                continue   # no pair, no rate
+            sk = engine.meanfield_simulate([ls], e_skew, steps, occ0[:1], record=record)
+            for g in (one, sk):
+                assert g.time[0] == pytest.approx(ref.time, rel=1e-10)
+                assert np.allclose(g.occupation[0, :N], ref.occupation, rtol=0, atol=1e-8)
+                assert np.allclose(g.electrode_occupation[0, :P], ref.electrode_occupation, rtol=1e-9, atol=1e-8)
+                assert np.allclose(g.site_energies[0, :N], ref.site_energies[:N], rtol=1e-9, atol=1e-9)
+                if record:
+                    assert np.allclose(g.average_occupation[0, :N], ref.average_occupation, rtol=1e-9,
+                                       atol=1e-8 * ref.time)
+                    assert np.allclose(g.traffic[0, :S, :S].ravel()[:S * S], ref.traffic.ravel(), rtol=1e-9, atol=1e-8)
+    finally:
+        for x in (lay, lb, ls):
+            x.close()
