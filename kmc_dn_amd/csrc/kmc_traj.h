@@ -761,19 +761,23 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
   // Kept transitions pay where trajectories come back to their states; one that
   // finds a new state on most hops would write records and bounds that nothing
   // reads.  So an interval with more than K / 2^kPlainShift new states is followed
-  // by kPlainIntervals intervals of general steps (and, where the energies follow
-  // from the occupation, ends with them).  20,000 hops of N = 30 (a = I_0 = 1,
+  // by general steps (and, where the energies follow from the occupation, ends with
+  // them): a spell of 2 intervals, of 8 if the interval after it finds as many
+  // again, then of kPlainIntervals, each over as soon as an interval
+  // of it evaluates fewer.  (Spells of 15 always: a trajectory whose first hops find many
+  // states spent most of 20,000 hops without leaps.)  20,000 hops of N = 30 (a = I_0 = 1,
   // nearly every hop new): alone 42.8 ms with transitions, 26.4 with this rule
   // (with two states and hops back only, 36.9); N = 56, 4096 of them 114.6, 78.3
   // (90.5).  At 1/2 instead of 1/4 the N = 56 network at 30 kT takes 62.3 ms
   // instead of 42.4; at 1/8 100,000 hops of the N = 30 network at 300 kT 32.3
   // instead of 26.4 ms.  Several chunks: at 1/8 a served population takes 27.4 ms
   // instead of 29.0 at 1/4.
-  constexpr int kPlainShift = kPathFree ? 2 : C == 1 ? 1 : 3, kPlainIntervals = 15;
+  constexpr int kPlainShift = kPathFree ? 2 : C == 1 ? 1 : 3, kPlainIntervals = 32;
   constexpr bool kSlowPrio = PRIO && ONE && T == 1;
   int nnew = in_vgpr_i(0);
   int slowv = in_vgpr_i(0);
-  int plainv = in_vgpr_i(0);   // intervals left that keep no transitions
+  // intervals left that keep no transitions, and (<< 8) the length of the next such spell
+  int plainv = in_vgpr_i(2 << 8);
   auto base_prio = [&]() __attribute__((always_inline)) {
     if constexpr (kSlowPrio) {
       if (__builtin_amdgcn_readfirstlane(slowv)) __builtin_amdgcn_s_setprio(2);
@@ -1510,6 +1514,12 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
       }
     }
   };
+  // A spell of general steps begins (more: intervals besides its length); the next
+  // one is four times as long.
+  auto next_spell = [&](int spell, int more) __attribute__((always_inline)) -> int {
+    const int n = spell >> 8;
+    return (n + more) | (n < kPlainIntervals ? 4 * n : n) << 8;
+  };
   // The work of a special hop before the hop itself: the clock's block sum,
   // uniforms, the end of the prehops, the FP64 recompute (which drops the kept
   // states and transitions).
@@ -1547,15 +1557,15 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
       pend = false;
       flush_tallies();
       drop_kept();
-      const int left = __builtin_amdgcn_readfirstlane(plainv);
+      const int spell = __builtin_amdgcn_readfirstlane(plainv), left = spell & 255;
+      const int nn = __builtin_amdgcn_readfirstlane(nnew);
       if (left > 0) {
-        plainv = in_vgpr_i(left - 1);
+        plainv = in_vgpr_i(nn > K >> kPlainShift ? spell - 1 : spell - left);
       } else {
-        const int nn = __builtin_amdgcn_readfirstlane(nnew);
         if constexpr (kSlowPrio) slowv = in_vgpr_i(nn > 16 ? 1 : 0);
-        plainv = in_vgpr_i(nn > K >> kPlainShift ? kPlainIntervals : 0);
-        nnew = in_vgpr_i(0);
+        plainv = in_vgpr_i(nn > K >> kPlainShift ? next_spell(spell, 0) : 2 << 8);
       }
+      nnew = in_vgpr_i(0);
       base_prio();
     } else if constexpr (kPathFree && !PH) {
       // (energies that follow from the occupation: no need to wait for the recompute)
@@ -1564,7 +1574,8 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
         flush_tallies();
         drop_kept();
         if constexpr (kSlowPrio) slowv = in_vgpr_i(1);
-        plainv = in_vgpr_i(kPlainIntervals + 1);
+        // (the rest of this interval besides)
+        plainv = in_vgpr_i(next_spell(__builtin_amdgcn_readfirstlane(plainv), 1));
         nnew = in_vgpr_i(0);
       }
     }
@@ -1748,6 +1759,7 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
         }
       }
       if (!cur_ok) {
+        if constexpr (!kGeneral) nnew = in_vgpr_i(nnew + 1);
         if constexpr (kPathFree) base_energies();
         else if (pend) rank1_energies(B.se);
         float R[C];
@@ -1811,7 +1823,7 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
   }
   while (!kGeneral && h < h_stop) {
     if (h == special && !special_work()) break;
-    if (__builtin_amdgcn_readfirstlane(plainv)) {
+    if (__builtin_amdgcn_readfirstlane(plainv) & 255) {
       general();
       if (status != ST_OK) break;
       continue;
