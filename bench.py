@@ -47,8 +47,8 @@ HBM_TRAFFIC_BYTES = 29_185_659
 # 4.096e8 hops), and the issue peak of each: one wave64 VALU instruction per 4 cycles on
 # each of a CU's 4 SIMDs, and one scalar instruction per cycle from the CU's shared
 # scalar unit, i.e. one per CU and cycle each, 256 CUs at 2.4 GHz.
-VALU_INSTS_PER_HOP = 6.25
-SALU_INSTS_PER_HOP = 5.77
+VALU_INSTS_PER_HOP = 4.14
+SALU_INSTS_PER_HOP = 3.84
 ISSUE_PEAK = 256 * 2.4e9
 
 
@@ -433,14 +433,12 @@ def main() -> int:
                                 if default_workload else None),
             "note": "achieved = algorithmic LDS bytes of the reference's dense formulation "
                     "(9,768 B per hop at N=30, P=8) x hops / kernel time; peak = ds_read_b128 "
-                    "stream measured in this run.  frac exceeds 1 because 97% of the hops never "
-                    "read those tables: a two-entry state cache serves 98.9% of the hops, an "
-                    "LDS store of evicted states most of the rest, and leaps take the runs of "
-                    "hops between the two cached states a whole uniform block at a time.  The "
-                    "launch ends with its slowest trajectories (those that hop among three or "
-                    "four states), bound by the latency of their hop chains (LdsUtil 3%, "
-                    "VALUBusy 34%, waves waiting on dependencies 41% of their cycles); "
-                    "valu/salu_issue_frac = profiled instructions per hop (6.25 VALU, 5.75 "
+                    "stream measured in this run.  frac exceeds 1 because most hops never read "
+                    "those tables: they are taken by kept transitions (one test of the hop's "
+                    "uniform), and runs between two states a whole uniform block at a time.  "
+                    "The launch ends with its slowest trajectories, bound by the latency of "
+                    "their hop chains; "
+                    "valu/salu_issue_frac = profiled instructions per hop (4.14 VALU, 3.84 "
                     "scalar) x hops / kernel time / (one per CU and cycle)",
         },
         "plain_fp64": {"value": plain_value, "unit": "hops/s",
