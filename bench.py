@@ -43,7 +43,7 @@ LDS_PEAK_SPEC_GBS = 256 * 256 * 2.4
 # I/O (1.1 MB) and register-spill scratch (the one-chunk kernels are held to 128 VGPRs).
 HBM_TRAFFIC_BYTES = 29_185_659
 # VALU and scalar instructions per hop and wave of the batched kernel on the default
-# workload (rocprofv3 --pmc SQ_INSTS_VALU 2.561e9, SQ_INSTS_SALU 2.362e9 per dispatch of
+# workload (rocprofv3 --pmc SQ_INSTS_VALU 1.695e9, SQ_INSTS_SALU 1.574e9 per dispatch of
 # 4.096e8 hops), and the issue peak of each: one wave64 VALU instruction per 4 cycles on
 # each of a CU's 4 SIMDs, and one scalar instruction per cycle from the CU's shared
 # scalar unit, i.e. one per CU and cycle each, 256 CUs at 2.4 GHz.
