@@ -71,11 +71,8 @@ kmc_batch_fp32_kernel(BatchParams p) {
 
 // Positions policy: every wave pulls its own groups and keeps only its layout's
 // site coordinates in LDS (at most 64*C float4), so a workgroup mixes layouts.
-// Over several chunks two waves share a SIMD: without the bound the three-chunk
-// kernel takes 296 VGPRs, one wave per SIMD, and of a batch of 2048 networks half wait
-// (the bench batch 1,065 ms, with the bound 1,042).
 template <int C, int W, bool REC>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(C == 1 ? 4 : 2)))
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(C == 1 ? 4 : 1)))
 kmc_batch_pos_kernel(BatchParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;

@@ -652,7 +652,10 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
   // by general steps: S = 129, 47 % new states 1.74 / 1.50; S = 112, 32 % 1.05 /
   // 0.84; S = 118, 15 % 0.55 / 0.60; S = 80, 0.4 % 0.17 / 0.37), and without the
   // tables their waves leave room on the SIMDs for a batch's other launches.
-  constexpr bool kGeneral = kMembers && C > 1;
+  // So do the positions kernels over several chunks, which serve the launches that
+  // fill the chip: with the tables they hold two waves per SIMD instead of three (the
+  // 2048 networks of the bench batch 1,042 ms, by general steps 975).
+  constexpr bool kGeneral = C > 1 && (kMembers || (T == 1 && !Pol::kElec));
   int psrc = 0, pdst = 0;
   bool pend = false;
   float base_se[C];
@@ -1755,7 +1758,7 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
             cur_ok = false;
             E0.val = E1.val = 0;
           }
-          special_work();
+          if (!special_work()) return false;
         }
       }
       if (!cur_ok) {
