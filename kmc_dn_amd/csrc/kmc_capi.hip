@@ -205,6 +205,10 @@ struct Batch {
     int32_t ngroups = 0;
     int smax = 0, nmax = 0, pmax = 0;
     bool split = false;   // one trajectory per group, for the kernels that split by site chunks
+    // the groups of a split entry for the runs that take its solo kernel after all (a
+    // grid limit, phase timing)
+    DevBuf whole;
+    int32_t nwhole = 0;
   };
   Sub subs[KMC_MAX_BUCKETS];
   bool subs_built = false;
@@ -1032,8 +1036,8 @@ int build_bucket_groups(Batch* B) {
   if (B->subs_built) return KMC_OK;
   Engine& E = eng();
   const int nb = (int)B->plan.size();
-  std::vector<std::vector<GroupDev>> g(nb);
   std::vector<int64_t> count(nb, 0);
+  bool any_split = false;
   for (int b = 0; b < nb; ++b) B->subs[b].smax = B->subs[b].nmax = B->subs[b].pmax = 0;
   auto bucket_at = [&](int64_t k) {
     const TrajDev& t = B->host[k];
@@ -1048,42 +1052,55 @@ int build_bucket_groups(Batch* B) {
     B->subs[b].nmax = std::max(B->subs[b].nmax, Ly->N);
     B->subs[b].pmax = std::max(B->subs[b].pmax, Ly->P);
   }
-  for (int b = 0; b < nb; ++b)
+  for (int b = 0; b < nb; ++b) {
     B->subs[b].split = B->plan[b].team <= 1 && B->plan[b].grid <= 0 &&
                        split_fits(count[b], B->plan[b].table_form, B->subs[b].smax,
                                   B->subs[b].nmax, B->subs[b].pmax);
-  int64_t i = 0;
-  while (i < B->ntraj) {
-    const Layout* Ly = E.layouts[B->host[i].layout];
-    const int b = bucket_at(i);
-    if (b < 0)
-      return fail(KMC_ERR_ARGS, "trajectory of layout %d (S=%d, budget %lld) matches no bucket",
-                  B->host[i].layout, Ly->S,
-                  (long long)(B->host[i].prehops + B->host[i].hops));
-    const kmc_bucket& pb = B->plan[b];
-    const int W =
-        (pb.table_form == 3 || pb.team > 1 || B->subs[b].split) ? 1 : pb.waves_per_group;
-    int64_t j = i;
-    while (j < B->ntraj && j - i < W && B->host[j].layout == B->host[i].layout && bucket_at(j) == b)
-      ++j;
-    GroupDev gd;
-    gd.layout = B->host[i].layout;
-    gd.first = (int32_t)i;
-    gd.count = (int32_t)(j - i);
-    gd.pad = 0;
-    g[b].push_back(gd);
-    i = j;
+    any_split = any_split || B->subs[b].split;
   }
-  for (int b = 0; b < nb; ++b) {
-    std::stable_sort(g[b].begin(), g[b].end(), [&](const GroupDev& x, const GroupDev& y) {
-      const TrajDev& u = B->host[x.first];
-      const TrajDev& v = B->host[y.first];
-      return u.prehops + u.hops > v.prehops + v.hops;
-    });
-    B->subs[b].ngroups = (int32_t)g[b].size();
-    int st = upload(B->subs[b].groups, g[b]);
-    if (st) return st;
-  }
+  // whole: the second set, of the split entries alone
+  auto build = [&](bool whole) -> int {
+    std::vector<std::vector<GroupDev>> g(nb);
+    int64_t i = 0;
+    while (i < B->ntraj) {
+      const Layout* Ly = E.layouts[B->host[i].layout];
+      const int b = bucket_at(i);
+      if (b < 0)
+        return fail(KMC_ERR_ARGS, "trajectory of layout %d (S=%d, budget %lld) matches no bucket",
+                    B->host[i].layout, Ly->S,
+                    (long long)(B->host[i].prehops + B->host[i].hops));
+      const kmc_bucket& pb = B->plan[b];
+      const bool one = pb.table_form == 3 || pb.team > 1 || (B->subs[b].split && !whole);
+      const int W = one ? 1 : pb.waves_per_group;
+      int64_t j = i;
+      while (j < B->ntraj && j - i < W && B->host[j].layout == B->host[i].layout &&
+             bucket_at(j) == b)
+        ++j;
+      GroupDev gd;
+      gd.layout = B->host[i].layout;
+      gd.first = (int32_t)i;
+      gd.count = (int32_t)(j - i);
+      gd.pad = 0;
+      g[b].push_back(gd);
+      i = j;
+    }
+    for (int b = 0; b < nb; ++b) {
+      Batch::Sub& sb = B->subs[b];
+      if (whole && !sb.split) continue;
+      std::stable_sort(g[b].begin(), g[b].end(), [&](const GroupDev& x, const GroupDev& y) {
+        const TrajDev& u = B->host[x.first];
+        const TrajDev& v = B->host[y.first];
+        return u.prehops + u.hops > v.prehops + v.hops;
+      });
+      (whole ? sb.nwhole : sb.ngroups) = (int32_t)g[b].size();
+      int st = upload(whole ? sb.whole : sb.groups, g[b]);
+      if (st) return st;
+    }
+    return KMC_OK;
+  };
+  int st = build(false);
+  if (!st && any_split) st = build(true);
+  if (st) return st;
   B->subs_built = true;
   return KMC_OK;
 }
@@ -1122,9 +1139,11 @@ int prepare_fp32(Batch* B, const kmc_run_opts& o, std::vector<Fp32Launch>& out,
       const kmc_bucket& pb = B->plan[b];
       if (pb.table_form == 3 && (st = check_positions(B, b))) return st;
       Fp32Launch L;
+      const bool split = sb.split && !phases && o.grid_limit <= 0;
+      const bool whole = sb.split && !split;
       st = setup_launch(B, o, pb.table_form, pb.waves_per_group, pb.team, sb.smax, sb.nmax,
-                        sb.pmax, sb.groups, sb.ngroups, q + 16 * b, pb.grid > 0 ? pb.grid : o.grid_limit, L,
-                        phases, sb.split && !phases && o.grid_limit <= 0);
+                        sb.pmax, whole ? sb.whole : sb.groups, whole ? sb.nwhole : sb.ngroups,
+                        q + 16 * b, pb.grid > 0 ? pb.grid : o.grid_limit, L, phases, split);
       if (st) return st;
       out.push_back(L);
     }
