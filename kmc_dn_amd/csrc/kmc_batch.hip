@@ -71,8 +71,14 @@ kmc_batch_fp32_kernel(BatchParams p) {
 
 // Positions policy: every wave pulls its own groups and keeps only its layout's
 // site coordinates in LDS (at most 64*C float4), so a workgroup mixes layouts.
+// Launches that fill the chip run these, so the waves a SIMD holds count: four of one
+// and two chunks (128 VGPRs, 15 to 26 spilled: the one-chunk code's tables), three of
+// three (168 VGPRs, 7 to 15 spilled).  Left to itself the compiler takes 173 VGPRs for
+// two chunks with records (two waves) and 218 to 227 for three (two): 3072 x 3000 hops of
+// S = 70 with records 7.8 ms, now 5.6; 3072 x 1000 of S = 148 6.0, now 4.5; without
+// records S = 70 at three waves 5.8, now 5.4.
 template <int C, int W, bool REC>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(C == 1 ? 4 : 1)))
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(C < 3 ? 4 : 3)))
 kmc_batch_pos_kernel(BatchParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;

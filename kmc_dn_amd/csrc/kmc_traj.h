@@ -653,8 +653,8 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
   // 0.84; S = 118, 15 % 0.55 / 0.60; S = 80, 0.4 % 0.17 / 0.37), and without the
   // tables their waves leave room on the SIMDs for a batch's other launches.
   // So do the positions kernels over several chunks, which serve the launches that
-  // fill the chip: with the tables they hold two waves per SIMD instead of three (the
-  // 2048 networks of the bench batch 1,042 ms, by general steps 975).
+  // fill the chip: the 2048 networks of the bench batch 1,042 ms with the tables, 975 by
+  // general steps (both at two waves per SIMD; kmc_batch_pos_kernel holds more now).
   constexpr bool kGeneral = C > 1 && (kMembers || (T == 1 && !Pol::kElec));
   int psrc = 0, pdst = 0;
   bool pend = false;
@@ -777,10 +777,14 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
   // instead of 29.0 at 1/4.
   constexpr int kPlainShift = kPathFree ? 2 : C == 1 ? 1 : 3, kPlainIntervals = 32;
   constexpr bool kSlowPrio = PRIO && ONE && T == 1;
-  int nnew = in_vgpr_i(0);
-  int slowv = in_vgpr_i(0);
+  int nnew = 0, slowv = 0;
   // intervals left that keep no transitions, and (<< 8) the length of the next such spell
-  int plainv = in_vgpr_i(2 << 8);
+  int plainv = 0;
+  if constexpr (!kGeneral) {
+    nnew = in_vgpr_i(0);
+    slowv = in_vgpr_i(0);
+    plainv = in_vgpr_i(2 << 8);
+  }
   auto base_prio = [&]() __attribute__((always_inline)) {
     if constexpr (kSlowPrio) {
       if (__builtin_amdgcn_readfirstlane(slowv)) __builtin_amdgcn_s_setprio(2);
@@ -1531,7 +1535,10 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
   // resumed range continues exactly as one long launch would).  The waves of a
   // team by members read their clocks apart and could disagree, so those carry no
   // limit (the host refuses one).
-  auto special_work = [&]() __attribute__((always_inline)) -> bool {
+  // empty: what else the recompute empties, here (the general steps' entries, reset
+  // ahead of this call, stayed live through the recompute: 30 to 44 VGPRs of the
+  // kernels over several chunks).
+  auto special_work = [&](auto empty) __attribute__((always_inline)) -> bool {
     if (!kMembers && p.time_limit > 0 && h == next_rc && h > h_begin) {
       bool over = wall_clock64() - t_start > p.time_limit;
       if constexpr (SPLIT) {
@@ -1558,17 +1565,20 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
       }
       next_rc = next_multiple(h);
       pend = false;
-      flush_tallies();
-      drop_kept();
-      const int spell = __builtin_amdgcn_readfirstlane(plainv), left = spell & 255;
-      const int nn = __builtin_amdgcn_readfirstlane(nnew);
-      if (left > 0) {
-        plainv = in_vgpr_i(nn > K >> kPlainShift ? spell - 1 : spell - left);
-      } else {
-        if constexpr (kSlowPrio) slowv = in_vgpr_i(nn > 16 ? 1 : 0);
-        plainv = in_vgpr_i(nn > K >> kPlainShift ? next_spell(spell, 0) : 2 << 8);
+      empty();
+      if constexpr (!kGeneral) {
+        flush_tallies();
+        drop_kept();
+        const int spell = __builtin_amdgcn_readfirstlane(plainv), left = spell & 255;
+        const int nn = __builtin_amdgcn_readfirstlane(nnew);
+        if (left > 0) {
+          plainv = in_vgpr_i(nn > K >> kPlainShift ? spell - 1 : spell - left);
+        } else {
+          if constexpr (kSlowPrio) slowv = in_vgpr_i(nn > 16 ? 1 : 0);
+          plainv = in_vgpr_i(nn > K >> kPlainShift ? next_spell(spell, 0) : 2 << 8);
+        }
+        nnew = in_vgpr_i(0);
       }
-      nnew = in_vgpr_i(0);
       base_prio();
     } else if constexpr (kPathFree && !PH) {
       // (energies that follow from the occupation: no need to wait for the recompute)
@@ -1753,13 +1763,11 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
     // starts with a recompute.
     auto step = [&](Entry& F, Entry& B) __attribute__((always_inline)) -> bool {
       if constexpr (kGeneral) {
-        if (__builtin_expect(h == special, 0)) {
-          if (h == next_rc) {
-            cur_ok = false;
-            E0.val = E1.val = 0;
-          }
-          if (!special_work()) return false;
-        }
+        if (__builtin_expect(h == special, 0) && !special_work([&]() __attribute__((always_inline)) {
+              cur_ok = false;
+              E0.val = E1.val = 0;
+            }))
+          return false;
       }
       if (!cur_ok) {
         if constexpr (!kGeneral) nnew = in_vgpr_i(nnew + 1);
@@ -1817,7 +1825,7 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
       if (!step(E0, E1)) break;
       if (!step(E1, E0)) break;
     }
-    drop_kept();
+    if constexpr (!kGeneral) drop_kept();
   };
 
   base_prio();
@@ -1825,7 +1833,7 @@ __device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, 
     if (h < h_stop) general();
   }
   while (!kGeneral && h < h_stop) {
-    if (h == special && !special_work()) break;
+    if (h == special && !special_work([] {})) break;
     if (__builtin_amdgcn_readfirstlane(plainv) & 255) {
       general();
       if (status != ST_OK) break;
