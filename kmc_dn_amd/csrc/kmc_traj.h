@@ -591,9 +591,13 @@ __device__ __forceinline__ uint64_t readlane_u64(uint64_t x, int l) {
 // one-chunk code of kernels over several chunks).
 // area: this wave's area of p.states.
 // polw: the pair terms of this wave's chunk alone (teams by site chunks).
+// Always inlined: out of line (as the compiler would have it for three chunks) the
+// policy's LDS pointers pass through memory, every table read is a generic load and
+// the kernel takes 256 VGPRs, 40 AGPRs and 750 bytes of scratch: 512 x 3000 hops of S =
+// 132 in table form 2, workgroups of four, 11.4 ms at 300 kT, inlined 8.3.
 template <int C, bool REC, class Pol, int T = 1, bool PRIO = true, bool PH = false,
           bool ONE = (C == 1), class TeamT = Team<T, C>, class PolW = Pol>
-__device__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, const Pol& pol,
+__device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, const LayoutDev& L, const Pol& pol,
                                int lane, const TeamT& team, unsigned char* area,
                                const PolW* polw = nullptr) {
   constexpr bool SPLIT = TeamT::kSplit;

@@ -77,3 +77,12 @@ def test_positions_kernels_hold_their_waves(kernels, chunks, waves):
     """Launches that fill the chip run these: 512 / VGPRs of them on a SIMD."""
     for name, k in _named(kernels, f"kmc_batch_pos_kernelILi{chunks}E").items():
         assert _waves_per_simd(k) >= waves, (name, k[".vgpr_count"])
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 3])
+def test_table_kernels_keep_their_hop_loop_inline(kernels, chunks):
+    """A hop loop called out of line reads its LDS tables by generic loads through
+    pointers in scratch (hundreds of bytes a lane; spills alone are within 200)."""
+    for name, k in _named(kernels, f"kmc_batch_fp32_kernelILi{chunks}E").items():
+        assert k[".private_segment_fixed_size"] <= 200, name
+        assert not k.get(".uses_dynamic_stack"), name
