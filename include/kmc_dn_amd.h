@@ -390,6 +390,11 @@ int kmc_probe_fp64_phases(int32_t batch, uint64_t* cycles, int32_t n);
  * the ordinary kernel's. */
 int kmc_probe_fp32_phases(int32_t batch, const kmc_run_opts* opts, uint64_t* cycles, int32_t n);
 
+/* Runs the batch as kmc_batch_run(batch, opts) would on the FP32 batched path, with
+ * every hop by a general step: no transition, state or run of hops is kept or looked
+ * up.  The same results, for comparison with the paths that keep them (no graph). */
+int kmc_probe_fp32_general(int32_t batch, const kmc_run_opts* opts);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1321,7 +1321,8 @@ int enqueue_fp64(Batch* B, const kmc_run_opts& o, hipStream_t s, const double* u
   return launch_plain(p, B->smax, B->nmax, rec, B->ntraj, s, B->queue.as<int32_t>(), nullptr, 0);
 }
 
-int batch_run_locked(int32_t id, const kmc_run_opts* opts) {
+// general: FP32 runs take general steps alone.
+int batch_run_locked(int32_t id, const kmc_run_opts* opts, bool general = false) {
   Engine& E = eng();
   Batch* B = get_batch(id);
   if (!B) return fail(KMC_ERR_ARGS, "bad batch id %d", id);
@@ -1357,6 +1358,8 @@ int batch_run_locked(int32_t id, const kmc_run_opts* opts) {
   }
   std::vector<Fp32Launch> Ls;
   if ((st = prepare_fp32(B, o, Ls))) return st;
+  if (general)
+    for (Fp32Launch& L : Ls) L.p.general_steps = 1;
   if (Ls.size() > 1 && (st = ensure_side_streams(B, (int)Ls.size()))) return st;
   if (o.use_graph) {
     // a graph replays its kernels' arguments as captured: re-capture when the
@@ -1729,6 +1732,19 @@ int kmc_probe_fp32_phases(int32_t batch, const kmc_run_opts* opts, uint64_t* cyc
   HIPOK(hipMemcpy(cycles, ph.p, sizeof(uint64_t) * FP32_PHASES, hipMemcpyDeviceToHost));
   B->last_rec = B->last_traffic = false;
   return KMC_OK;
+}
+
+int kmc_probe_fp32_general(int32_t batch, const kmc_run_opts* opts) {
+  Engine& E = eng();
+  std::lock_guard<std::mutex> lk(E.mu);
+  int st = ensure_init();
+  if (st) return st;
+  if (opts && (opts->precision != KMC_FP32_BATCHED || opts->use_graph))
+    return fail(KMC_ERR_UNSUPPORTED, "general steps: FP32 batched runs without a graph");
+  kmc_run_opts o{};
+  if (opts) o = *opts;
+  o.precision = KMC_FP32_BATCHED;
+  return batch_run_locked(batch, &o, true);
 }
 
 int kmc_batch_destroy(int32_t batch) {

@@ -780,6 +780,7 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
   // instead of 26.4 ms.  Several chunks: at 1/8 a served population takes 27.4 ms
   // instead of 29.0 at 1/4.
   constexpr int kPlainShift = kPathFree ? 2 : C == 1 ? 1 : 3, kPlainIntervals = 32;
+  constexpr int kAlways = 255;   // a spell that does not end (p.general_steps)
   constexpr bool kSlowPrio = PRIO && ONE && T == 1;
   int nnew = 0, slowv = 0;
   // intervals left that keep no transitions, and (<< 8) the length of the next such spell
@@ -787,7 +788,7 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
   if constexpr (!kGeneral) {
     nnew = in_vgpr_i(0);
     slowv = in_vgpr_i(0);
-    plainv = in_vgpr_i(2 << 8);
+    plainv = in_vgpr_i((p.general_steps ? kAlways : 0) | 2 << 8);
   }
   auto base_prio = [&]() __attribute__((always_inline)) {
     if constexpr (kSlowPrio) {
@@ -1579,7 +1580,7 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
         const int spell = __builtin_amdgcn_readfirstlane(plainv), left = spell & 255;
         const int nn = __builtin_amdgcn_readfirstlane(nnew);
         if (left > 0) {
-          plainv = in_vgpr_i(nn > K >> kPlainShift ? spell - 1 : spell - left);
+          if (left != kAlways) plainv = in_vgpr_i(nn > K >> kPlainShift ? spell - 1 : spell - left);
         } else {
           if constexpr (kSlowPrio) slowv = in_vgpr_i(nn > 16 ? 1 : 0);
           plainv = in_vgpr_i(nn > K >> kPlainShift ? next_spell(spell, 0) : 2 << 8);
