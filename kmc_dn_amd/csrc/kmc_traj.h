@@ -767,19 +767,24 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
   // longest trajectories (3.5 % longer).  No result depends on it.
   // Kept transitions pay where trajectories come back to their states; one that
   // finds a new state on most hops would write records and bounds that nothing
-  // reads.  So an interval with more than K / 2^kPlainShift new states is followed
-  // by general steps (and, where the energies follow from the occupation, ends with
-  // them): a spell of 2 intervals, of 8 if the interval after it finds as many
-  // again, then of kPlainIntervals, each over as soon as an interval
-  // of it evaluates fewer.  (Spells of 15 always: a trajectory whose first hops find many
+  // reads.  So an interval ends by general steps once it has found more than K /
+  // 2^kPlainShift new states (tested every 64 hops), and a spell of them follows: 2
+  // intervals, 8 if the interval after it finds as many again, then
+  // kPlainIntervals, each over as soon as an interval
+  // of it evaluates fewer (the rest of the one it began in counts as many).  Where the
+  // energies follow from the path, the last two states pass on as the general steps'
+  // entries (until this did, such an interval ran to its end with transitions: 512 x
+  // 4000 hops of S = 109 with records, nearly every hop new, 11.2 ms, now 9.0).  (Spells of 15 always: a trajectory whose first hops find many
   // states spent most of 20,000 hops without leaps.)  20,000 hops of N = 30 (a = I_0 = 1,
   // nearly every hop new): alone 42.8 ms with transitions, 26.4 with this rule
   // (with two states and hops back only, 36.9); N = 56, 4096 of them 114.6, 78.3
   // (90.5).  At 1/2 instead of 1/4 the N = 56 network at 30 kT takes 62.3 ms
   // instead of 42.4; at 1/8 100,000 hops of the N = 30 network at 300 kT 32.3
   // instead of 26.4 ms.  Several chunks: at 1/8 a served population takes 27.4 ms
-  // instead of 29.0 at 1/4.
-  constexpr int kPlainShift = kPathFree ? 2 : C == 1 ? 1 : 3, kPlainIntervals = 32;
+  // instead of 29.0 at 1/4; at 1/16 S = 109 gains 1 to 3 % and 600 trajectories of S =
+  // 148 at 300 kT lose 10.  One-chunk teams, S = 58 at 1 / 300 kT: 1/4 0.92 / 2.84 ms,
+  // 1/8 0.92 / 2.61, 1/16 1.15 / 2.46.
+  constexpr int kPlainShift = kPathFree ? 2 : 3, kPlainIntervals = 32;
   constexpr int kAlways = 255;   // a spell that does not end (p.general_steps)
   constexpr bool kSlowPrio = PRIO && ONE && T == 1;
   int nnew = 0, slowv = 0;
@@ -1588,16 +1593,16 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
         nnew = in_vgpr_i(0);
       }
       base_prio();
-    } else if constexpr (kPathFree && !PH) {
-      // (energies that follow from the occupation: no need to wait for the recompute)
+    } else if constexpr (!kGeneral && !PH) {
       if (__builtin_amdgcn_readfirstlane(nnew) > K >> kPlainShift) {
         current_occ();
         flush_tallies();
-        drop_kept();
+        if constexpr (kPathFree) drop_kept();
         if constexpr (kSlowPrio) slowv = in_vgpr_i(1);
         // (the rest of this interval besides)
         plainv = in_vgpr_i(next_spell(__builtin_amdgcn_readfirstlane(plainv), 1));
-        nnew = in_vgpr_i(0);
+        // (the interval has found that many, whatever its rest evaluates)
+        nnew = in_vgpr_i((K >> kPlainShift) + 1);
       }
     }
     special = next_special(h, false);
@@ -1607,7 +1612,8 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
   };
 
   // The hops up to the next recompute by general steps, which keep the current
-  // state and the one before it, in registers, and no transitions.  The entries
+  // state and the one before it, in registers, and no transitions.  Within an interval,
+  // where the energies follow from the path, they go on from the kept ones.  The entries
   // swap roles on every hop; the loop is unrolled by two hops, one for each
   // assignment of the roles, so a hop back moves no data.  (The tables of kept
   // states and transitions hold nothing here, and no registers.)
@@ -1766,6 +1772,54 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
     Entry E0, E1;
     E0.val = E1.val = 0;
     bool cur_ok = false;   // the current state's entry holds it
+    // The prefix over F's rows R, its total and what follows from them into F;
+    // false: no rate is positive and finite.
+    auto sums = [&](Entry& F, const float (&R)[C]) __attribute__((always_inline)) -> bool {
+      double total = 0.0;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        if (c > 0 && 64 * c >= S) {
+          F.inc[c] = F.exc[c] = total;
+          F.nzr[c] = in_vgpr((uint64_t)0);
+          continue;
+        }
+        F.inc[c] = c == 0 ? wave_scan_f64((double)R[c]) : wave_scan_f64((double)R[c]) + total;
+        F.exc[c] = F.inc[c] - (double)R[c];
+        F.nzr[c] = in_vgpr(ballot(R[c] > 0.f));
+        total = readlane_f64(F.inc[c], 63);
+      }
+      F.tot = in_vgpr(total);
+      F.rtot = __builtin_amdgcn_rcpf((float)total);
+      F.psel = -2;
+      F.val = 1;
+      return total > 0.0 && total < INFINITY;
+    };
+    if constexpr (!kGeneral && !kPathFree) {
+      // kept state k into F
+      auto hand_over = [&](Entry& F, int k) __attribute__((always_inline)) {
+        float R[C];
+        int nocc = 0;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          F.key[c] = readlane_u64(key[c], k);
+          nocc += popcount64(F.key[c] & accm[c]);
+          R[c] = k == rid ? rrow[c] : prow[c];
+          F.se[c] = k == rid ? rse[c] : pse[c];
+          if (k != rid && k != pid) {
+            R[c] = c > 0 && 64 * c >= S ? 0.f : rec(k)[64 * c];
+            F.se[c] = c > 0 && 64 * c >= S ? 0.f : rec(k)[64 * (C + c)];
+          }
+        }
+        F.udst = N - nocc <= nocc;
+        (void)sums(F, R);
+      };
+      if (prev >= 0) hand_over(E1, prev);
+      if (cur >= 0) {
+        hand_over(E0, cur);
+        cur_ok = true;
+      }
+      drop_kept();
+    }
     // One hop whose current state's entry is F (B: the entry of the state
     // before); false: the trajectory stops here, its range ends or the next hop
     // starts with a recompute.
@@ -1783,28 +1837,14 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
         else if (pend) rank1_energies(B.se);
         float R[C];
         F.udst = evaluate(R);
-        // FP64 prefix over lane rows
-        double total = 0.0;
 #pragma unroll
         for (int c = 0; c < C; ++c) {
           F.key[c] = occ[c];
           F.se[c] = se[c];
-          if (c > 0 && 64 * c >= S) {
-            F.inc[c] = F.exc[c] = total;
-            F.nzr[c] = in_vgpr((uint64_t)0);
-            continue;
-          }
-          F.inc[c] = c == 0 ? wave_scan_f64((double)R[c]) : wave_scan_f64((double)R[c]) + total;
-          F.exc[c] = F.inc[c] - (double)R[c];
-          F.nzr[c] = in_vgpr(ballot(R[c] > 0.f));
-          total = readlane_f64(F.inc[c], 63);
         }
-        F.tot = in_vgpr(total);
-        F.rtot = __builtin_amdgcn_rcpf((float)total);
-        F.psel = -2;
-        F.val = 1;
+        const bool ok = sums(F, R);
         mark(2);
-        if (!(total > 0.0 && total < INFINITY)) {
+        if (!ok) {
           status = ST_ZERO_RATE;
           return false;
         }
