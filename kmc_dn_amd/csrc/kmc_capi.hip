@@ -204,9 +204,10 @@ struct Batch {
     DevBuf groups;
     int32_t ngroups = 0;
     int smax = 0, nmax = 0, pmax = 0;
+    int64_t ntraj = 0;
     bool split = false;   // one trajectory per group, for the kernels that split by site chunks
     // the groups of a split entry for the runs that take its solo kernel after all (a
-    // grid limit, phase timing)
+    // grid limit, phase timing, records where those workgroups do not fit)
     DevBuf whole;
     int32_t nwhole = 0;
   };
@@ -906,20 +907,28 @@ BatchKernel pick_split_kernel(int C, bool rec, int form) {
 
 // Whether a solo launch over `ntraj` trajectories of layouts with at most S, N
 // and P sites gives each of them a wave per site chunk (kmc_split_kernel, the
-// same bits): while all of those waves fit beside each other, two on a SIMD (their
-// registers' limit; table forms: a workgroup on a CU, their LDS's).  10,000 hops,
-// ms solo / split: S = 148 in the positions form, 64 trajectories 30.7 / 13.7, 512
-// 47.1 / 21.1, 680 47.2 / 29.3 (1024 do not fit); S = 78, 64 of them 1.70 / 1.55, 1024
-// 6.79 / 6.11; S = 109 in table form 2, 256 of them 10.3 / 9.8, all states new 23.1 /
-// 20.5.
-constexpr int SPLIT_WAVES_PER_CU = 8;
-bool split_fits(int64_t ntraj, int form, int smax, int nmax, int pmax) {
+// same bits): while all of their workgroups fit beside each other, by the kernel's own
+// registers and LDS (positions form: four a CU of two chunks, two of three; table forms:
+// one).  One that waited would double the launch: S = 148 in the positions form, 2500
+// hops, nearly every one new, ms solo / split: 64 trajectories 17.3 / 10.7, 480 17.6 /
+// 12.2, 560 (three workgroups of three waves do not fit) 17.5 / 21.6; 4000 hops at 1 kT
+// 10.8 / 7.7, 11.4 / 9.1, 11.5 / 12.3.  S = 109, 1024 of them, 10.2 / 9.5 and 7.3 / 6.6; in
+// table form 2, 256 of them, 5.4 / 4.9 and 3.3 / 3.2.  S = 78, 1024 of them, 4000 hops
+// at 1 kT 4.6 / 3.4.
+bool split_fits(int64_t ntraj, int form, int smax, int nmax, int pmax, bool rec) {
   const int C = (smax + 63) / 64;
-  if (C < 2) return false;
-  if (form != 3 && (ntraj > eng().cu_count ||
-                    split_lds_bytes(form, C, smax, nmax, pmax) > (size_t)160 * 1024))
+  // (at most two waves on a SIMD, by their registers)
+  if (C < 2 || ntraj * C > 8 * (int64_t)eng().cu_count) return false;
+  const size_t lds = split_lds_bytes(form, C, smax, nmax, pmax);
+  if (lds > (size_t)160 * 1024) return false;
+  const void* k = (const void*)pick_split_kernel(C, rec, form);
+  int per_cu = 0;
+  if (!k || hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64 * C, lds) != hipSuccess) {
+    (void)hipGetLastError();
     return false;
-  return ntraj * C <= SPLIT_WAVES_PER_CU * (int64_t)eng().cu_count;
+  }
+  return ntraj <= (int64_t)per_cu * eng().cu_count;
 }
 
 struct Fp32Launch {
@@ -1036,9 +1045,9 @@ int build_bucket_groups(Batch* B) {
   if (B->subs_built) return KMC_OK;
   Engine& E = eng();
   const int nb = (int)B->plan.size();
-  std::vector<int64_t> count(nb, 0);
   bool any_split = false;
-  for (int b = 0; b < nb; ++b) B->subs[b].smax = B->subs[b].nmax = B->subs[b].pmax = 0;
+  for (int b = 0; b < nb; ++b)
+    B->subs[b].ntraj = B->subs[b].smax = B->subs[b].nmax = B->subs[b].pmax = 0;
   auto bucket_at = [&](int64_t k) {
     const TrajDev& t = B->host[k];
     return bucket_of(B, E.layouts[t.layout]->S, t.prehops + t.hops);
@@ -1047,15 +1056,15 @@ int build_bucket_groups(Batch* B) {
     const Layout* Ly = E.layouts[B->host[k].layout];
     const int b = bucket_at(k);
     if (b < 0) continue;   // (refused below)
-    ++count[b];
+    ++B->subs[b].ntraj;
     B->subs[b].smax = std::max(B->subs[b].smax, Ly->S);
     B->subs[b].nmax = std::max(B->subs[b].nmax, Ly->N);
     B->subs[b].pmax = std::max(B->subs[b].pmax, Ly->P);
   }
   for (int b = 0; b < nb; ++b) {
     B->subs[b].split = B->plan[b].team <= 1 && B->plan[b].grid <= 0 &&
-                       split_fits(count[b], B->plan[b].table_form, B->subs[b].smax,
-                                  B->subs[b].nmax, B->subs[b].pmax);
+                       split_fits(B->subs[b].ntraj, B->plan[b].table_form, B->subs[b].smax,
+                                  B->subs[b].nmax, B->subs[b].pmax, false);
     any_split = any_split || B->subs[b].split;
   }
   // whole: the second set, of the split entries alone
@@ -1129,6 +1138,7 @@ int prepare_fp32(Batch* B, const kmc_run_opts& o, std::vector<Fp32Launch>& out,
                  uint64_t* phases = nullptr) {
   int st = prepare_record(B, o);
   if (st) return st;
+  const bool rec = (o.record & 3) != 0;
   int32_t* q = B->queue.as<int32_t>();
   if (!B->plan.empty()) {
     if ((st = build_bucket_groups(B))) return st;
@@ -1139,7 +1149,8 @@ int prepare_fp32(Batch* B, const kmc_run_opts& o, std::vector<Fp32Launch>& out,
       const kmc_bucket& pb = B->plan[b];
       if (pb.table_form == 3 && (st = check_positions(B, b))) return st;
       Fp32Launch L;
-      const bool split = sb.split && !phases && o.grid_limit <= 0;
+      const bool split = sb.split && !phases && o.grid_limit <= 0 &&
+                         (!rec || split_fits(sb.ntraj, pb.table_form, sb.smax, sb.nmax, sb.pmax, rec));
       const bool whole = sb.split && !split;
       st = setup_launch(B, o, pb.table_form, pb.waves_per_group, pb.team, sb.smax, sb.nmax,
                         sb.pmax, whole ? sb.whole : sb.groups, whole ? sb.nwhole : sb.ngroups,
@@ -1161,7 +1172,7 @@ int prepare_fp32(Batch* B, const kmc_run_opts& o, std::vector<Fp32Launch>& out,
   if (team != 1 && team != 2 && team != 4) return fail(KMC_ERR_ARGS, "team must be 1, 2 or 4");
   if (form == 3 && (st = check_positions(B, -1))) return st;
   const bool split = team <= 1 && !phases && o.grid_limit <= 0 &&
-                     split_fits(B->ntraj, form, B->smax, B->nmax, B->pmax);
+                     split_fits(B->ntraj, form, B->smax, B->nmax, B->pmax, rec);
   // positions, teams and splits: one trajectory per group
   if ((st = build_groups(B, (form == 3 || team > 1 || split) ? 1 : W))) return st;
   Fp32Launch L;
