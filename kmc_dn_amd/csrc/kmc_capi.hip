@@ -1245,7 +1245,10 @@ int launch_fp32(Batch* B, const kmc_run_opts& o, const std::vector<Fp32Launch>& 
 
 // State records of the FP64 kernel: at most this much device memory for all
 // workgroups of a launch, and at most PLAIN_SLOTS_MAX per workgroup (one
-// trajectory at +-300 kT visits 500 to 2000 states in 2e4 hops).
+// trajectory at +-300 kT visits 500 to 2000 states in 2e4 hops), as long as the tags'
+// LDS (16 B a record) keeps beside each other the workgroups that 64 records would.
+// 4000 hops of N = 30, P = 8 at +-300 kT, 255 trajectories 4.53 ms, 257 with 64 records 6.64,
+// with 512 4.53; 700 of them 7.49 and, with 128, 5.96.
 constexpr size_t PLAIN_STATES_MAX = (size_t)512 << 20;
 constexpr int PLAIN_SLOTS_MAX = 1024;
 
@@ -1275,12 +1278,23 @@ int launch_plain(PlainParams p, int S, int N, bool rec, int64_t ntraj, hipStream
   int64_t grid = ntraj;
   int slots = PLAIN_SLOTS_MAX;
   if (ntraj > E.cu_count) {
-    slots = 64;
-    const size_t lds = plain_lds_bytes(S, N, slots, stage);
-    int per_cu = 0;
-    HIPOK(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    HIPOK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, 64, lds));
-    grid = std::min<int64_t>(ntraj, (int64_t)std::max(1, per_cu) * E.cu_count);
+    auto resident = [&](int n, int& per_cu) -> hipError_t {
+      const size_t lds = plain_lds_bytes(S, N, n, stage);
+      per_cu = 0;
+      if (lds > cap) return hipSuccess;
+      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      return e != hipSuccess ? e
+                             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, 64, lds);
+    };
+    int per_cu = 0, with = 0;
+    HIPOK(resident(64, per_cu));
+    per_cu = std::max(1, per_cu);
+    grid = std::min<int64_t>(ntraj, (int64_t)per_cu * E.cu_count);
+    const int need = (int)((grid + E.cu_count - 1) / E.cu_count);
+    for (; slots > 64; slots /= 2) {
+      HIPOK(resident(slots, with));
+      if (with >= need) break;
+    }
   }
   while (slots > 1 && plain_lds_bytes(S, N, slots, stage) > cap) slots /= 2;
   const size_t most = states ? nstates : PLAIN_STATES_MAX;

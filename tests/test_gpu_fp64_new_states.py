@@ -7,7 +7,7 @@ import pytest
 
 import oracle
 from kmc_dn_amd import _lib, engine
-from tests.netgen import random_network
+from tests.netgen import fixture_network, random_network
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +50,25 @@ def test_new_states_cost_little_besides_their_evaluation(gpu_engine):
     b.close()
     lay.close()
     assert sum(c[4:]) < sum(c[:4]) / 7, list(c)
+
+
+def test_records_beyond_a_trajectory_per_cu(gpu_engine, fixtures):
+    """One trajectory fewer than CUs and two more, of a fixture network at +-300 kT: as many
+    records each (64 instead, and the evicted states evaluated again, take 1.5 times
+    as long)."""
+    net = fixture_network(fixtures, "rnd", 4)
+    lay = engine.Layout(30, 8, net["nu"], net["kT"], net["I_0"], net["R"], net["distances"], net["transitions_constant"])
+    es = lay.energy_sets(net["E_constant"], net["site_energies"][30:])
+    cus = engine.device_info()["cu_count"]
+    ms = []
+    for K in (cus - 1, cus + 2):
+        b = engine.Batch(engine.make_trajs(K, lay.id, int(es[0]), np.arange(K, dtype=np.uint64), 4000, net["occupation"]))
+        print(f"[gpu] FP64 records: {K} trajectories", flush=True)
+        took = []
+        for _ in range(3):
+            b.run(precision=_lib.FP64_DENSE)
+            took.append(b.sync())
+        ms.append(min(took[1:]))
+        b.close()
+    lay.close()
+    assert ms[1] < 1.2 * ms[0], ms
