@@ -149,6 +149,7 @@ struct DevBuf {
     if (bytes == 0) return KMC_OK;
     hipError_t e = hipMalloc(&p, bytes);
     if (e != hipSuccess) {
+      (void)hipGetLastError();   // (the caller is told; no later launch's check is to see it)
       p = nullptr;
       n = cap = 0;
       return fail(KMC_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
@@ -246,8 +247,8 @@ struct Engine {
   // PLAIN_STATES_MAX bytes; freed by kmc_reset)
   DevBuf plain_states;
   // state records of the FP32 kernels' resident waves (32 KiB per wave and site
-  // chunk, at most 16 waves of one chunk or 12 of three per CU: 300 MB a launch;
-  // freed by kmc_reset)
+  // chunk of the code that keeps states, at most 16 waves of one chunk or 8 of three
+  // per CU: 200 MB a launch; freed by kmc_reset)
   DevBuf states;
   std::vector<Batch*> batches;
   bool layouts_dirty = true, esets_dirty = true;
@@ -1014,7 +1015,10 @@ int setup_launch(Batch* B, const kmc_run_opts& o, int form, int W, int team, int
   p.time_limit = o.time_limit_us > 0 ? (int64_t)o.time_limit_us * E.wall_khz / 1000 : 0;
   // a positive state_store: the two last states and that many more
   p.state_slots = o.state_store == 0 ? STATE_SLOTS : 2 + std::max(0, o.state_store);
-  p.state_area = (int64_t)C * STATE_SLOTS * STATE_RECORD_BYTES;
+  // site chunks of the code that keeps states: none in teams by members over several
+  // chunks, the one-chunk code alone in the positions kernels
+  const int kept = team > 1 ? (C == 1 ? 1 : 0) : form == 3 && !split ? 1 : C;
+  p.state_area = (int64_t)kept * STATE_SLOTS * STATE_RECORD_BYTES;
   L.k = k;
   L.grid = grid;
   L.block = 64 * W;
@@ -1117,25 +1121,30 @@ int build_bucket_groups(Batch* B) {
 // The launches' state records in the engine's buffer: every run of every batch is
 // ordered on the engine stream, and the launches of one run have areas of
 // their own.  A captured graph holds the addresses: reg_gen tells it when they move.
-int place_states(std::vector<Fp32Launch>& Ls) {
+// Without that memory (and with `general`) the launches take general steps, which keep
+// no states: the same bits.
+void place_states(std::vector<Fp32Launch>& Ls, bool general) {
   Engine& E = eng();
   size_t need = 0;
   for (const Fp32Launch& L : Ls) need += (size_t)L.grid * (L.block / 64) * L.p.state_area;
-  const void* was = E.states.p;
-  int st = E.states.alloc(need);
-  if (E.states.p != was) ++E.reg_gen;
-  if (st) return st;
-  unsigned char* at = E.states.as<unsigned char>();
+  if (!general && need > 0) {
+    const void* was = E.states.p;
+    general = E.states.alloc(need) != KMC_OK;
+    if (E.states.p != was) ++E.reg_gen;
+  }
+  unsigned char* at = general ? nullptr : E.states.as<unsigned char>();
   for (Fp32Launch& L : Ls) {
+    L.p.general_steps = general ? 1 : 0;
+    if (general) L.p.state_area = 0;
     L.p.states = at;
     at += (size_t)L.grid * (L.block / 64) * L.p.state_area;
   }
-  return KMC_OK;
 }
 
 // Everything that allocates or queries happens here, outside any graph capture.
+// general: general steps alone.
 int prepare_fp32(Batch* B, const kmc_run_opts& o, std::vector<Fp32Launch>& out,
-                 uint64_t* phases = nullptr) {
+                 uint64_t* phases = nullptr, bool general = false) {
   int st = prepare_record(B, o);
   if (st) return st;
   const bool rec = (o.record & 3) != 0;
@@ -1158,7 +1167,8 @@ int prepare_fp32(Batch* B, const kmc_run_opts& o, std::vector<Fp32Launch>& out,
       if (st) return st;
       out.push_back(L);
     }
-    return place_states(out);
+    place_states(out, general);
+    return KMC_OK;
   }
   const int C = (B->smax + 63) / 64;
   int form = o.table_form;
@@ -1180,7 +1190,8 @@ int prepare_fp32(Batch* B, const kmc_run_opts& o, std::vector<Fp32Launch>& out,
                          o.grid_limit, L, phases, split)))
     return st;
   out.push_back(L);
-  return place_states(out);
+  place_states(out, general);
+  return KMC_OK;
 }
 
 int launch_one(const Fp32Launch& L, hipStream_t s) {
@@ -1382,9 +1393,7 @@ int batch_run_locked(int32_t id, const kmc_run_opts* opts, bool general = false)
     if (team) return fail(KMC_ERR_UNSUPPORTED, "time limits apply to solo kernels only (team > 1)");
   }
   std::vector<Fp32Launch> Ls;
-  if ((st = prepare_fp32(B, o, Ls))) return st;
-  if (general)
-    for (Fp32Launch& L : Ls) L.p.general_steps = 1;
+  if ((st = prepare_fp32(B, o, Ls, nullptr, general))) return st;
   if (Ls.size() > 1 && (st = ensure_side_streams(B, (int)Ls.size()))) return st;
   if (o.use_graph) {
     // a graph replays its kernels' arguments as captured: re-capture when the

@@ -109,7 +109,9 @@ class Server:
     chunk_hops: sets the round's target device time, chunk_hops x 1.5 us; each
       trajectory's hop range per round is that time over its measured seconds per
       hop (a multiple of the recompute interval).
-    max_active / mem_budget: trajectory slots and device bytes of admitted state.
+    max_active / mem_budget: trajectory slots and device bytes of admitted state (the
+      kernels' state records, at most 32 KiB per resident wave and site chunk, come
+      besides; without room for them the rounds run slower, with the same results).
     team_min_hops: budgets from which a request runs in a team bucket (None: solo
       buckets only; every admitted trajectory must be resident in each round, and
       table-form teams hold a CU's LDS each).
