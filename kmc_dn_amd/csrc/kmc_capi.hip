@@ -819,9 +819,20 @@ int build_groups(Batch* B, int W) {
     const TrajDev& y = B->host[b.first];
     return x.prehops + x.hops > y.prehops + y.hops;
   });
+  // a run with other groups may still read the ones that this replaces
+  if (B->group_mode != -1) HIPOK(hipStreamSynchronize(eng().stream));
+  B->group_mode = -1;
+  const void* was = B->groups.p;
+  int st = upload(B->groups, g);
+  // a captured graph holds their address
+  if (B->graph && B->groups.p != was) {
+    (void)hipGraphExecDestroy(B->graph);
+    B->graph = nullptr;
+  }
+  if (st) return st;
   B->ngroups = (int32_t)g.size();
   B->group_mode = W;
-  return upload(B->groups, g);
+  return KMC_OK;
 }
 
 int bucket_of(const Batch* B, int S, int64_t budget) {
