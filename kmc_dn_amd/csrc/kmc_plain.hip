@@ -46,7 +46,7 @@
 //    their tags alone over the next block, selects the events from the prefix sums
 //    and stores a record when a tag comes back.  2000 hops of N = 30, P = 8, nearly every
 //    one new (a = I_0 = 1): 19.7 ms with every record stored, now 18.0 (16.6 with no
-//    records at all); at +-300 kT 1.76 and 1.80 (10.0).
+//    records at all); at +-300 kT 1.76 and 1.78 (9.9).
 //  * A run of hops back and forth between two states (a leap).  Whether the hop
 //    with event uniform u leads from A to B depends on u alone: lo < u <= hi,
 //    the quotients around the event.  The lanes test the 64 hops of a uniform
@@ -100,8 +100,9 @@ __device__ __forceinline__ int div_small(int x, int d, float rcp, int& r) {
 
 // A state's tag: the occupation (acceptors 0-63 in the first word, 64-79 in the
 // low bits of the second), bit 63 of the second word set, its kept entries
-// above bit 32 (none: a state that was seen and has no record).
+// above bit 32.  Bit 62 instead of 63: a state that was seen and has no record.
 constexpr uint64_t TAG_VALID = 1ull << 63;
+constexpr uint64_t TAG_SEEN = 1ull << 62;
 constexpr uint64_t TAG_STATE = TAG_VALID | 0xFFFFull;
 
 // State records of one workgroup: {1/total, total}, then the quotients of the
@@ -400,6 +401,16 @@ __device__ __forceinline__ void plain_trajectory(const PlainParams& p, const int
     return way;
   };
 
+  // The way of the current state's tag without a record in set `set` (-1: not seen).
+  // (Asked of new states only: a test of the looked-up tag for both kinds cost hops from
+  // recorded states 5 %.)
+  auto seen_way = [&]() -> int {
+    const ulonglong2 tg =
+        *reinterpret_cast<const ulonglong2*>(tags + 2 * (set * ways + (lane & (ways - 1))));
+    const uint64_t m = ballot(tg.x == occ0 && tg.y == (occ1 | TAG_SEEN));
+    return m ? __builtin_ctzll(m) & (ways - 1) : -1;
+  };
+
   // The hop before the current one: where it started, its event and bounds.  A
   // hop that undoes it makes (state before, current state) a pair, whose two
   // events the leap tests.
@@ -457,11 +468,11 @@ __device__ __forceinline__ void plain_trajectory(const PlainParams& p, const int
     prev = !first;
     mark(6);
   };
-  // A tag for the current state in set `set`, its record of n entries (0: none).
-  auto tag = [&](int way, int n) __attribute__((always_inline)) {
+  // A tag for the current state in set `set`: `mark` its second word's upper bits.
+  auto tag = [&](int way, uint64_t mark) __attribute__((always_inline)) {
     if (lane == 0) {
       tags[2 * (set * ways + way)] = occ0;
-      tags[2 * (set * ways + way) + 1] = occ1 | TAG_VALID | ((uint64_t)n << 32);
+      tags[2 * (set * ways + way) + 1] = occ1 | mark;
     }
   };
   // A hop of the current state, which has no tag: the tag alone is set and the event
@@ -473,7 +484,7 @@ __device__ __forceinline__ void plain_trajectory(const PlainParams& p, const int
     if (total == 0.0) return false;
     const int way = __builtin_amdgcn_readfirstlane(next_way[set]);
     if (lane == 0) next_way[set] = (way + 1) & (ways - 1);
-    tag(way, 0);
+    tag(way, TAG_SEEN);
     const double ue = readlane_f64(ue_lane, h & 63), scale = 1.0 / total;
     double lo = 0.0, hi = 0.0;
     int code = -1;
@@ -578,7 +589,8 @@ __device__ __forceinline__ void plain_trajectory(const PlainParams& p, const int
     }
     // the state's record: read, or evaluated and stored first
     int way = lookup();
-    if (way < 0 || ns == 0) {
+    if (way < 0) {
+      way = seen_way();
       const bool seen = way >= 0;
       if (!seen) ++fresh;
       if (!seen && tags_only) {
@@ -602,7 +614,7 @@ __device__ __forceinline__ void plain_trajectory(const PlainParams& p, const int
         way = __builtin_amdgcn_readfirstlane(next_way[set]);
         if (lane == 0) next_way[set] = (way + 1) & (ways - 1);
       }
-      tag(way, ns);
+      tag(way, TAG_VALID | ((uint64_t)ns << 32));
       const StateRecord r = record(set * ways + way);
       double* q = r.quot();
       uint16_t* ev = r.event(p.npairs);
