@@ -305,7 +305,11 @@ kmc_meanfield_kernel(MeanfieldParams p) {
 // probSimulate for the networks that kmc_meanfield_kernel does not take: the table
 // of a larger one does not fit in LDS, and with asymmetric tables the terms that a
 // row and a column see differ.  The terms out of and into every site go through
-// LDS in tiles of MF_TILE partners; the same bits.
+// LDS in tiles of MF_TILE partners; the same bits.  One such network sends a call's
+// every network here (a launch has one kernel): 64 networks of 28 to 108 sites, 100 steps
+// with records, 4.5 ms a call for an asymmetric table instead of 1.8 (25.6 with one
+// wave per network); with one of 158 sites 7.7, which is that network's own time (16 of
+// them 7.0; 56 and 59 with one wave each).
 constexpr int MF_TILE_WAVES = 16;
 template <int C>
 __global__ void __launch_bounds__(64 * MF_TILE_WAVES) kmc_meanfield_tiled_kernel(MeanfieldParams p) {

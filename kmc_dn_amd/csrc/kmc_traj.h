@@ -581,7 +581,7 @@ __device__ __forceinline__ uint64_t readlane_u64(uint64_t x, int l) {
 // leaps) and now: 4096 x 1e5 hops of N = 30 at 1 kT 44.9 and 15.3 ms; one
 // trajectory of 1e5 hops with records 63.4 and 9.1 ms, at 300 kT 47.7 and 26.4
 // ms; 4096 x 2e4 hops of an IV sweep 10.0 and 3.7 ms; 64 x 21,000 of N = 100
-// with records 25.9 and 22.6 ms.
+// with records 25.9 and 18.1 ms.
 //
 // PH: the phase-timing instantiation: shader-clock reads at the phase
 // boundaries of every hop (FP32_PHASES), summed into p.phases by the first wave
@@ -1065,53 +1065,52 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
     return v;
   };
 
-  // Energies of the state with occupation occ from the last recompute's.
+  // Energies of the state with occupation occ from the last recompute's: those plus the
+  // Coulomb columns of the acceptors whose occupation differs from the recompute's
+  // (+ where now occupied, - where now empty), added in ascending site order; the
+  // columns of up to G sites are loaded together (a site past the last loads the
+  // first's column and adds nothing).
   auto base_energies = [&]() __attribute__((always_inline)) {
     if constexpr (kPathFree) {
-              // its energies: the recompute's plus the Coulomb columns of the
-              // acceptors whose occupation differs from the recompute's (+ where
-              // now occupied, - where now empty), added in ascending site order;
-              // the columns of up to G sites are loaded together (a site past the
-              // last loads the first's column and adds nothing)
-              constexpr int G = 8;
-              se[0] = base_se[0];
-              uint64_t dm = (occ[0] ^ base_occ[0]) & accm[0];
-              while (dm) {
-                int js[G];
-                const int j0 = __builtin_ctzll(dm);
-      #pragma unroll
-                for (int g = 0; g < G; ++g) {
-                  js[g] = dm ? __builtin_ctzll(dm) : -1;
-                  dm &= dm - 1;
-                }
-                float cv[G];
-      #pragma unroll
-                for (int g = 0; g < G; ++g) cv[g] = pol.coul(js[g] < 0 ? j0 : js[g], 0);
-      #pragma unroll
-                for (int g = 0; g < G; ++g) {
-                  if (js[g] < 0) break;
-                  const bool on = (occ[0] >> js[g]) & 1ull;
-                  se[0] += on ? cv[g] : -cv[g];
-                }
-              }
+      constexpr int G = 8;
+      se[0] = base_se[0];
+      uint64_t dm = (occ[0] ^ base_occ[0]) & accm[0];
+      while (dm) {
+        int js[G];
+        const int j0 = __builtin_ctzll(dm);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          js[g] = dm ? __builtin_ctzll(dm) : -1;
+          dm &= dm - 1;
+        }
+        float cv[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) cv[g] = pol.coul(js[g] < 0 ? j0 : js[g], 0);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          if (js[g] < 0) break;
+          const bool on = (occ[0] >> js[g]) & 1ull;
+          se[0] += on ? cv[g] : -cv[g];
+        }
+      }
     }
   };
   // ... from the energies of the state before it.
   auto rank1_energies = [&](const float (&bse)[C]) __attribute__((always_inline)) {
-          const bool src_acc = psrc < N, dst_acc = pdst < N;
-          float cs[C], cd[C];
-    #pragma unroll
-          for (int c = 0; c < C; ++c) {
-            if constexpr (Pol::kZeroColumnN) {   // column N holds c = 0: no select per lane
-              cs[c] = (c == 0 || 64 * c < S) ? pol.coul(min((unsigned)psrc, (unsigned)N), c) : 0.f;
-              cd[c] = (c == 0 || 64 * c < S) ? pol.coul(min((unsigned)pdst, (unsigned)N), c) : 0.f;
-            } else {
-              cs[c] = (c == 0 || 64 * c < S) && src_acc ? pol.coul(psrc, c) : 0.f;
-              cd[c] = (c == 0 || 64 * c < S) && dst_acc ? pol.coul(pdst, c) : 0.f;
-            }
-          }
-    #pragma unroll
-          for (int c = 0; c < C; ++c) se[c] = (bse[c] - cs[c]) + cd[c];
+    const bool src_acc = psrc < N, dst_acc = pdst < N;
+    float cs[C], cd[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if constexpr (Pol::kZeroColumnN) {   // column N holds c = 0: no select per lane
+        cs[c] = (c == 0 || 64 * c < S) ? pol.coul(min((unsigned)psrc, (unsigned)N), c) : 0.f;
+        cd[c] = (c == 0 || 64 * c < S) ? pol.coul(min((unsigned)pdst, (unsigned)N), c) : 0.f;
+      } else {
+        cs[c] = (c == 0 || 64 * c < S) && src_acc ? pol.coul(psrc, c) : 0.f;
+        cd[c] = (c == 0 || 64 * c < S) && dst_acc ? pol.coul(pdst, c) : 0.f;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) se[c] = (bse[c] - cs[c]) + cd[c];
   };
 
   // The current state (occupation occ) looked up or evaluated; false: it has no
@@ -1894,7 +1893,7 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
       }
       // hops of this uniform block from kept states
       while (h < h_lim && cur >= 0) {
-          if (tryleap) {
+        if (tryleap) {
           const int n = leap();
           tryleap = n > 0 && h == h_lim;   // the block's end, not the run's, ended it
           mark(6);

@@ -152,10 +152,10 @@ constexpr int STORE_MAX_SLOTS = 4;   // largest kmc_run_opts.state_store
 // terms, row sums and team reduction of a new state (or its lookup), 2 its FP64
 // prefix scan and record, 3 event selection of a new transition, 4 its partner
 // selection, 5 its insertion and the hop, 6 hops by kept transitions and leaps
-// (general steps: 0 to 5); slot 7 counts the
-// hops from a state that the hop before led back into, slot 8 those by a kept
-// transition (general steps: by a partner prefix formed before), slot 9 those taken by leaps, slot 10 the states found among the
-// kept ones instead of evaluated.
+// (general steps: 0 to 5).  Slot 7 counts the hops from a state that the hop before
+// led back into, slot 8 those by a kept transition (general steps: by a partner
+// prefix formed before), slot 9 those taken by leaps, slot 10 the states found
+// among the kept ones instead of evaluated.
 constexpr int FP32_PHASES = 11;
 
 struct PlainParams {
