@@ -1145,7 +1145,6 @@ void place_states(std::vector<Fp32Launch>& Ls, bool general) {
   }
   unsigned char* at = general ? nullptr : E.states.as<unsigned char>();
   for (Fp32Launch& L : Ls) {
-    L.p.general_steps = general ? 1 : 0;
     if (general) L.p.state_area = 0;
     L.p.states = at;
     at += (size_t)L.grid * (L.block / 64) * L.p.state_area;

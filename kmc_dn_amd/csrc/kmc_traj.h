@@ -589,7 +589,7 @@ __device__ __forceinline__ uint64_t readlane_u64(uint64_t x, int l) {
 // loads, so its hops are somewhat slower than the others'.
 // ONE: the code runs in a kernel built for one site chunk (false for the
 // one-chunk code of kernels over several chunks).
-// area: this wave's area of p.states.
+// area: this wave's area of p.states; null: general steps alone.
 // polw: the pair terms of this wave's chunk alone (teams by site chunks).
 // Always inlined: out of line (as the compiler would have it for three chunks) the
 // policy's LDS pointers pass through memory, every table read is a generic load and
@@ -785,7 +785,7 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
   // 148 at 300 kT lose 10.  One-chunk teams, S = 58 at 1 / 300 kT: 1/4 0.92 / 2.84 ms,
   // 1/8 0.92 / 2.61, 1/16 1.15 / 2.46.
   constexpr int kPlainShift = kPathFree ? 2 : 3, kPlainIntervals = 32;
-  constexpr int kAlways = 255;   // a spell that does not end (p.general_steps)
+  constexpr int kAlways = 255;   // a spell that does not end (no area)
   constexpr bool kSlowPrio = PRIO && ONE && T == 1;
   int nnew = 0, slowv = 0;
   // intervals left that keep no transitions, and (<< 8) the length of the next such spell
@@ -793,7 +793,7 @@ __device__ __forceinline__ void run_trajectory(const BatchParams& p, int t, cons
   if constexpr (!kGeneral) {
     nnew = in_vgpr_i(0);
     slowv = in_vgpr_i(0);
-    plainv = in_vgpr_i((p.general_steps ? kAlways : 0) | 2 << 8);
+    plainv = in_vgpr_i((area ? 0 : kAlways) | 2 << 8);
   }
   auto base_prio = [&]() __attribute__((always_inline)) {
     if constexpr (kSlowPrio) {

@@ -135,8 +135,9 @@ struct BatchParams {
                                 // it stops at its next recompute point; 0: none
   int32_t state_slots;          // states a one-chunk solo trajectory keeps, 2..STATE_SLOTS
                                 // (the others: STATE_SLOTS)
-  int32_t general_steps;        // 1: general steps alone, which touch no state records
-  unsigned char* states;        // the waves' state records, state_area bytes per wave
+  int32_t pad2;
+  unsigned char* states;        // the waves' state records, state_area bytes per wave; null
+                                // (and state_area 0): general steps alone
   int64_t state_area;
 };
 
