@@ -37,18 +37,19 @@ METRIC = "hops/sec, 4096-traj N=30 ensemble vs plain; p50/p99 latency of served 
 # divides by the LDS read peak measured in the same run (ds_read_b128 stream probe).
 LDS_PEAK_SPEC_GBS = 256 * 256 * 2.4
 # HBM bytes per launch of the batched kernel on the default workload (4096 x 1e5 hops,
-# N=30/P=8, auto table form and workgroup size): rocprofv3 --pmc FETCH_SIZE 5738.81 KiB
-# and WRITE_SIZE 17024 KiB per dispatch, scaled by the copy-kernel calibration factors
-# 2.0 (FETCH) and 1.0 (WRITE): (2 * 5738.81 + 17024) * 1024 bytes -- the launch's own
-# I/O (1.1 MB) and register-spill scratch (the one-chunk kernels are held to 128 VGPRs).
-HBM_TRAFFIC_BYTES = 29_185_659
+# N=30/P=8, auto table form and workgroup size): rocprofv3 --pmc FETCH_SIZE 18016.9 KiB
+# and WRITE_SIZE 145285 KiB per dispatch, scaled by the copy-kernel calibration factors
+# 2.0 (FETCH) and 1.0 (WRITE): (2 * 18016.9 + 145285) * 1024 bytes -- the kept states'
+# records, register-spill scratch (the one-chunk kernels are held to 128 VGPRs) and the
+# launch's own I/O (1.1 MB).
+HBM_TRAFFIC_BYTES = 185_670_451
 # VALU and scalar instructions per hop and wave of the batched kernel on the default
-# workload (rocprofv3 --pmc SQ_INSTS_VALU 1.695e9, SQ_INSTS_SALU 1.574e9 per dispatch of
+# workload (rocprofv3 --pmc SQ_INSTS_VALU 1.710e9, SQ_INSTS_SALU 1.576e9 per dispatch of
 # 4.096e8 hops), and the issue peak of each: one wave64 VALU instruction per 4 cycles on
 # each of a CU's 4 SIMDs, and one scalar instruction per cycle from the CU's shared
 # scalar unit, i.e. one per CU and cycle each, 256 CUs at 2.4 GHz.
-VALU_INSTS_PER_HOP = 4.14
-SALU_INSTS_PER_HOP = 3.84
+VALU_INSTS_PER_HOP = 4.18
+SALU_INSTS_PER_HOP = 3.85
 ISSUE_PEAK = 256 * 2.4e9
 
 
@@ -438,7 +439,7 @@ def main() -> int:
                     "uniform), and runs between two states a whole uniform block at a time.  "
                     "The launch ends with its slowest trajectories, bound by the latency of "
                     "their hop chains; "
-                    "valu/salu_issue_frac = profiled instructions per hop (4.14 VALU, 3.84 "
+                    "valu/salu_issue_frac = profiled instructions per hop (4.18 VALU, 3.85 "
                     "scalar) x hops / kernel time / (one per CU and cycle)",
         },
         "plain_fp64": {"value": plain_value, "unit": "hops/s",

@@ -369,8 +369,9 @@ int kmc_probe_chain(int kind, int iters, double* cycles_per_instruction);
 /* Runs the batch once on the FP64 dense kernel's phase-timing instantiation
  * (shader-clock reads at the phase boundaries of every hop, same work) and
  * returns trajectory 0's shader cycles summed per phase: cycles[0..6] =
- * energies, pair lists, rates, prefix chain, uniforms and clock, event search,
- * hop and records (n >= 7). */
+ * a new state's energies, pair lists (and the lookup before), rates, prefix chain,
+ * record (or, without one, event); event search of recorded states; hops, runs of
+ * hops, uniforms and clock (n >= 7). */
 int kmc_probe_fp64_phases(int32_t batch, uint64_t* cycles, int32_t n);
 
 /* Runs the batch once as kmc_batch_run(batch, opts) would on the FP32 batched

@@ -61,7 +61,7 @@ def lone(N: int, P: int, form: int, team: int, hops: int = 20_000, seed: int = 1
             "us_per_hop": ms * 1e3 / hops}
 
 
-FP64_PHASES = ["energies", "pair_lists", "rates", "prefix_chain", "uniforms_clock", "search",
+FP64_PHASES = ["energies", "pair_lists", "rates", "prefix_chain", "records", "search",
                "hop_records"]
 
 
